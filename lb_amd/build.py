@@ -50,6 +50,8 @@ def _run(cmd, cwd=None):
 
 
 CORE_UNITS = ["lbm_core.hip", "closure.hip", "voxel.hip", "noalloc.hip"]
+# steps.hip is compiled once per storage policy (storage.hpp)
+STORES = ["StoreF64", "StoreF32", "StoreF16Dev", "StoreBF16Dev", "StoreF16DevSR", "StoreBF16DevSR"]
 
 
 def build_core():
@@ -60,6 +62,10 @@ def build_core():
         obj = os.path.join(CSRC, u.replace(".hip", ".o"))
         objs.append(obj)
         jobs.append([HIPCC, *HIP_FLAGS, "-c", "-o", obj, src])
+    for st in STORES:
+        obj = os.path.join(CSRC, f"steps_{st}.o")
+        objs.append(obj)
+        jobs.insert(0, [HIPCC, *HIP_FLAGS, f"-DLBM_STORE={st}", "-c", "-o", obj, os.path.join(CSRC, "steps.hip")])
     with ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
         list(ex.map(_run, jobs))
     out = os.path.join(HERE, "liblbm_core_hip.so")

@@ -18,417 +18,43 @@
 #include <vector>
 
 #include "../../include/lbm_closure.h"
-#include "lbm_kernels.hpp"
+#include "context.hpp"
 
 using namespace lbm;
 
 // closure.hip: BF16 inference image of a parameter vector
 void lbm_mlp_pack_bf16(const float* p, uint16_t* w1, uint16_t* w2);
 
-struct lbm_ctx {
-    lbm_desc d;
-    int device = 0;
-    hipStream_t stream = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    size_t N = 0;              // padded cells
-    size_t NU = 0;             // caller's cells
-    size_t elem = 0;           // bytes per stored population
-    size_t rbytes = 0;         // bytes per arithmetic value
-    Geo g{};
-    bool flags_needed = false; // any non-fluid cell (halo included)
-    int n_inlet = 0, n_eq = 0, n_outlet = 0, n_ghost = 0, n_pub = 0;
-    int n_upd = 0;                // moving-wall and Zou-He inlet entries
-    std::vector<int> ghost_off;  // launch boundaries of the ghost list (dependency levels)
-    void* pops = nullptr;
-    uint8_t* cls = nullptr;
-    uint64_t* node = nullptr;
-    int32_t* bcidx = nullptr;
-    void* inl_state = nullptr;
-    NodeDev* inl = nullptr;
-    NodeDev* outl = nullptr;
-    NodeDev* ghost = nullptr;
-    void* pub_mac = nullptr;
-    void* inl_post = nullptr;     // hand-over to the inlet rule (k_inlet_state, or deferred): f* and rho, u
-    void* inl_mac = nullptr;
-    void* pub_post = nullptr;
-    void* macro = nullptr;     // 4 planes, arithmetic type, padded layout
-    double* stage = nullptr;   // 5 planes FP64, caller layout
-    double* partials = nullptr;
-    std::vector<double> h_partials;
-    int64_t steps = 0;
-    bool initialized = false;
-    bool first = false;
-    bool nan_seen = false;
-    bool diag_next = false;    // the next launched step reduces mass, momentum and wall force
-    double last_ms = 0.0;
-    size_t dev_bytes = 0;
-    // learned closure
-    bool mlp_ready = false;
-    float* cl_params = nullptr;   // FP32 parameters
-    uint16_t* cl_wb = nullptr;    // BF16 W1 [64][16] + W2 [64][64]
-    float cl_b3 = 0.0f;
-    float* cl_norm = nullptr;     // [4][12] mean, 1/sd, envelope low, high
-    float* ccache = nullptr;      // coefficient per cell held between network evaluations
-    int cl_every = 1;             // evaluate the network every cl_every steps
-    int64_t cl_count = 0;         // steps since the last (re)start of the refresh cycle
-    // time averaging (MomentTimeAvg)
-    double* avg = nullptr;        // 4 FP64 planes, caller layout: sums of rho, ux, uy, uz
-    int64_t avg_count = 0;        // states added
-    bool avg_pending = false;     // the current state is counted but not yet added
-    bool avg_each = false;        // launch_steps: count the state after every step
-    // probe records taken without a synchronisation
-    double* probe_buf = nullptr;  // [PROBE_CAP][4] on the device
-    int probe_n = 0;              // records in probe_buf
-    std::vector<double> probe_host;  // records drained from the device, oldest first
-    // outlet omega damping
-    int sp_axis = -1, sp_begin = 0, sp_interval = 1;
-    // ErrorQuadratic on the device
-    std::vector<uint8_t> h_flag1;   // flag == 1 per caller cell (the cells the norm sums over)
-    uint8_t* flag1 = nullptr;       // the same on the device, uploaded by the first evaluation
-    void* uerr = nullptr;           // previous velocity, 3 planes of the arithmetic type, caller layout
-    // per-block partials of a diagnostics step go here instead of `partials` when set
-    double* diag_dst = nullptr;
-    // asynchronous snapshots: rho, u, omega into snap_dev on the context stream,
-    // then a copy to pinned host memory on copy_stream while steps go on
-    double* snap_dev = nullptr;       // 5 planes FP64, caller layout
-    double* snap_host = nullptr;      // pinned, 5 planes
-    hipStream_t copy_stream = nullptr;
-    hipEvent_t ev_snap = nullptr, ev_snap_copy = nullptr;
-    bool snap_pending = false;
-    int64_t snap_step = 0;
-    // Deferred interpolated outlet: the rule runs in the next reader of an
-    // outlet cell, with the post-collision records of the step that produced
-    // the state.  Records alternate between pub_post (even steps) and
-    // pub_post2 (odd steps), so a step can read the previous step's while
-    // writing its own.
-    bool outl_deferred = false;
-    bool outl_pending = false;      // the current state's outlet cells still need the rule
-    void* pub_post2 = nullptr;
-    // Deferred inlet: the moving-wall and Zou-He rules run in the next
-    // step's kernel from the records (inl_post, inl_mac) of the step that
-    // produced the state.
-    bool inl_deferred = false;
-    bool inl_pending = false;       // the inlet cells' stored state still needs its rule
-};
-
-static constexpr int PROBE_CAP = 4096;
-
-// The interpolated outlet's weight c_s = 1/sqrt(3) (OutletDensityInterpolated.h:226)
-// in the constants' precision.
-template <class R>
-static R outlet_cs(const lbm_ctx* c)
+// Sum of nb per-block partial records (stride doubles apart, ncomp <= 8
+// components each) into out[0 .. ncomp), by one workgroup in a fixed order:
+// thread t adds records t, t + 256, ... in turn, then a tree over the
+// threads.  Deterministic for a given nb.
+__global__ __launch_bounds__(TPB) void k_reduce_partials(const double* parts, int nb, int stride, int ncomp,
+                                                         double* out)
 {
-    return (c->d.compat & LBM_COMPAT_F32CONST) ? (R)(1.f / sqrtf(3.f)) : (R)(1.0 / std::sqrt(3.0));
-}
-
-// Post-collision records written by step t (deferred outlet: alternating buffers).
-static void* pub_records(const lbm_ctx* c, int64_t t)
-{
-    return (c->outl_deferred && (t & 1)) ? c->pub_post2 : c->pub_post;
-}
-
-#define HIPCHK(x)                                   \
-    do {                                            \
-        hipError_t e_ = (x);                        \
-        if (e_ != hipSuccess) return LBM_E_HIP;     \
-    } while (0)
-
-static lbm_status dev_alloc(lbm_ctx* c, void** p, size_t bytes)
-{
-    if (bytes == 0) bytes = 16;
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        *p = nullptr;
-        return LBM_E_OOM;
+    __shared__ double red[TPB][8];
+    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int b = (int)threadIdx.x; b < nb; b += TPB)
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (k < ncomp) acc[k] += parts[(size_t)b * stride + k];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) red[threadIdx.x][k] = acc[k];
+    __syncthreads();
+    for (int h = TPB / 2; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) red[threadIdx.x][k] += red[threadIdx.x + h][k];
+        __syncthreads();
     }
-    c->dev_bytes += bytes;
-    return LBM_OK;
+    if ((int)threadIdx.x < ncomp) out[threadIdx.x] = red[0][threadIdx.x];
 }
 
-template <class ST>
-static void fill_common(const lbm_ctx* c, typename ST::T** p, typename ST::R* rest, Consts<typename ST::R>& K)
+// Plain stream copy used as the bandwidth reference.
+__global__ __launch_bounds__(TPB) void k_copy(const float4* __restrict__ src, float4* __restrict__ dst, size_t n)
 {
-    using R = typename ST::R;
-    K = make_consts<R>(c->d.compat);
-    for (int k = 0; k < 4; ++k) rest[k] = ST::dev ? (R)(K.w[k] * (R)c->d.rho0) : R(0);
-    typename ST::T* base = (typename ST::T*)c->pops;
-    for (int q = 0; q < Q; ++q) p[q] = base + (size_t)q * c->N;
-}
-
-static MlpWeights closure_weights(const lbm_ctx* c)
-{
-    MlpWeights W;
-    W.w1 = c->cl_wb;
-    W.w2 = c->cl_wb ? c->cl_wb + NHID * 16 : nullptr;
-    W.b1 = c->cl_params ? c->cl_params + OFF_B1 : nullptr;
-    W.b2 = c->cl_params ? c->cl_params + OFF_B2 : nullptr;
-    W.w3 = c->cl_params ? c->cl_params + OFF_W3 : nullptr;
-    W.norm = c->cl_norm;
-    W.b3 = c->cl_b3;
-    W.c = (float)c->d.c_les;
-    return W;
-}
-
-template <class ST>
-static AuxArgs<ST> aux_args(const lbm_ctx* c)
-{
-    using R = typename ST::R;
-    AuxArgs<ST> a;
-    std::memset(&a, 0, sizeof(a));
-    fill_common<ST>(c, a.p, a.rest, a.K);
-    a.cls = c->cls;
-    a.bcidx = c->bcidx;
-    a.inl_state = (R*)c->inl_state;
-    a.macro = (R*)c->macro;
-    a.g = c->g;
-    a.tau = (R)c->d.tau;
-    a.cles = (R)c->d.c_les;
-    a.omega0 = R(1) / (R)c->d.tau;
-    a.closure = c->d.closure;
-    a.lit = c->d.arith == LBM_ARITH_LITERAL;
-    a.odd = (int)(c->steps & 1);
-    a.first = c->first ? 1 : 0;
-    a.io = c->stage;
-    a.sp_axis = c->sp_axis;
-    a.sp_begin = c->sp_begin;
-    a.sp_deriv = ((R)c->d.sponge_high - (R)c->d.sponge_low) / (R)c->sp_interval;
-    a.outl_pending = c->outl_pending ? 1 : 0;
-    a.outl = c->outl;
-    a.pub_prev = (const R*)pub_records(c, c->steps - 1);
-    a.cs = outlet_cs<R>(c);
-    a.crev20 = (c->d.compat & LBM_COMPAT_CREV20) ? 1 : 0;
-    a.inl_pending = c->inl_pending ? 1 : 0;
-    a.inl = c->inl;
-    a.inl_post = (const R*)c->inl_post;
-    a.inl_mac = (const R*)c->inl_mac;
-    return a;
-}
-
-static unsigned blocks_for(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
-
-template <class ST>
-static PatchArgs<ST> patch_args(const lbm_ctx* c)
-{
-    using R = typename ST::R;
-    PatchArgs<ST> a;
-    std::memset(&a, 0, sizeof(a));
-    fill_common<ST>(c, a.p, a.rest, a.K);
-    a.cls = c->cls;
-    a.bcidx = c->bcidx;
-    a.inl_state = (R*)c->inl_state;
-    a.pub_mac = (const R*)c->pub_mac;
-    a.pub_post = (const R*)c->pub_post;
-    a.g = c->g;
-    a.nu = (R)c->d.nu;
-    // the outlet's interpolation weight (OutletDensityInterpolated.h:226) is
-    // 1/sqrt(3) in the constants' precision
-    a.cs = outlet_cs<R>(c);
-    a.inletrho = (c->d.compat & LBM_COMPAT_INLETRHO) ? 1 : 0;
-    a.crev20 = (c->d.compat & LBM_COMPAT_CREV20) ? 1 : 0;
-    return a;
-}
-
-// Boundary rules that read what other cells produced in the same step, in
-// the reference's order: inlet, outlet, periodic.
-template <class ST>
-static lbm_status launch_patches(lbm_ctx* c, int odd_next)
-{
-    PatchArgs<ST> a = patch_args<ST>(c);
-    a.odd = odd_next;
-    a.pub_post = (const typename ST::R*)pub_records(c, c->steps);   // this step's records
-    if (c->n_upd && !c->inl_deferred) {
-        PatchArgs<ST> u = a;
-        u.nodes = c->inl;
-        u.n = c->n_inlet;
-        u.pub_mac = (const typename ST::R*)c->inl_mac;
-        u.pub_post = (const typename ST::R*)c->inl_post;
-        k_inlet_state<ST><<<blocks_for(u.n), TPB, 0, c->stream>>>(u);
-    }
-    if (c->n_eq) {
-        a.nodes = c->inl;
-        a.n = c->n_inlet;
-        k_inlet_eq<ST><<<blocks_for(a.n), TPB, 0, c->stream>>>(a);
-    }
-    if (c->n_outlet && !c->outl_deferred) {
-        a.nodes = c->outl;
-        a.n = c->n_outlet;
-        k_outlet<ST><<<blocks_for(a.n), TPB, 0, c->stream>>>(a);
-    }
-    for (size_t l = 0; l + 1 < c->ghost_off.size(); ++l) {
-        a.nodes = c->ghost + c->ghost_off[l];
-        a.n = c->ghost_off[l + 1] - c->ghost_off[l];
-        k_periodic<ST><<<blocks_for(a.n), TPB, 0, c->stream>>>(a);
-    }
-    HIPCHK(hipGetLastError());
-    return LBM_OK;
-}
-
-// Add the pending state to the time-average sums with its own pass.
-template <class ST>
-static lbm_status avg_flush_st(lbm_ctx* c)
-{
-    if (!c->avg_pending) return LBM_OK;
-    AuxArgs<ST> a = aux_args<ST>(c);
-    a.io = c->avg;
-    k_moment_add<ST><<<blocks_for(c->NU), TPB, 0, c->stream>>>(a);
-    HIPCHK(hipGetLastError());
-    c->avg_pending = false;
-    return LBM_OK;
-}
-
-// Seed of the stochastic-rounding stores of step t (any fixed bijective mix
-// of the step counter: runs with the same inputs give the same results).
-static uint32_t step_seed(uint64_t t)
-{
-    uint64_t x = t * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
-    x ^= x >> 31;
-    x *= 0xBF58476D1CE4E5B9ull;
-    x ^= x >> 27;
-    return (uint32_t)(x >> 32);
-}
-
-// The boundary-aware step: 16-bit storage takes the kernel held to 7 waves
-// per SIMD, the other formats the plain entry point.
-template <class ST, int COLL, bool LIT, bool ODD, bool INL>
-static void launch_flagged(dim3 grid, dim3 block, hipStream_t s, const StepArgs<ST>& a)
-{
-    if constexpr (sizeof(typename ST::T) == 2)
-        k_step_w7<ST, COLL, LIT, ODD, INL><<<grid, block, 0, s>>>(a);
-    else
-        k_step<ST, COLL, LIT, ODD, true, false, INL><<<grid, block, 0, s>>>(a);
-}
-
-template <class ST, int COLL, bool LIT>
-static lbm_status launch_steps(lbm_ctx* c, int nsteps)
-{
-    using R = typename ST::R;
-    StepArgs<ST> a;
-    std::memset(&a, 0, sizeof(a));
-    fill_common<ST>(c, a.p, a.rest, a.K);
-    a.cls = c->cls;
-    a.node = c->node;
-    a.bcidx = c->bcidx;
-    a.inl_state = (R*)c->inl_state;
-    a.inl = c->inl;
-    a.pub_mac = (R*)c->pub_mac;
-    a.pub_post = (R*)c->pub_post;
-    a.inl_post = (R*)c->inl_post;
-    a.inl_mac = (R*)c->inl_mac;
-    a.macro = (const R*)c->macro;
-    a.partials = c->diag_dst ? c->diag_dst : c->partials;
-    a.ccache = c->ccache;
-    a.g = c->g;
-    a.sp_axis = c->sp_axis;
-    a.sp_begin = c->sp_begin;
-    a.sp_deriv = ((R)c->d.sponge_high - (R)c->d.sponge_low) / (R)c->sp_interval;
-    a.outl = c->outl;
-    a.cs = outlet_cs<R>(c);
-    a.omega0 = R(1) / (R)c->d.tau;   // 1.f / tau (OmegaNo.h:44, NonDim...h:114)
-    a.tau = (R)c->d.tau;
-    a.cles = (R)c->d.c_les;
-    a.crev20 = (c->d.compat & LBM_COMPAT_CREV20) ? 1 : 0;
-    a.closure = c->d.closure;
-    const bool mlp = c->d.closure == LBM_CLOSURE_MLP;
-    MlpStepArgs<ST> ma;
-    if (mlp) {
-        if (!c->mlp_ready) return LBM_E_STATE;
-        ma.mlp = closure_weights(c);
-    }
-    const bool patches = (c->n_upd && !c->inl_deferred) || c->n_eq || (c->n_outlet && !c->outl_deferred) ||
-                         c->n_ghost;
-    const dim3 grid((unsigned)c->g.ntiles), block(TPB);
-    HIPCHK(hipEventRecord(c->ev0, c->stream));
-    for (int s = 0; s < nsteps; ++s) {
-        a.first = c->first ? 1 : 0;
-        // a counted state is added by the step that reads it; the network step
-        // does not fuse the add, so it gets its own pass first
-        if (mlp && c->avg_pending && c->cl_count % c->cl_every == 0) {
-            lbm_status st = avg_flush_st<ST>(c);
-            if (st != LBM_OK) return st;
-        }
-        a.avg = c->avg_pending ? c->avg : nullptr;
-        c->avg_pending = false;
-        a.diag = (s == 0 && c->diag_next) ? 1 : 0;
-        a.pub_post = (R*)pub_records(c, c->steps);
-        a.pub_prev = (const R*)pub_records(c, c->steps - 1);
-        a.outl_pending = c->outl_pending ? 1 : 0;
-        a.inl_pending = c->inl_pending ? 1 : 0;
-        if constexpr (ST::sr) a.seed = step_seed((uint64_t)c->steps);
-        const bool odd = (c->steps & 1) != 0;
-        if constexpr (sizeof(R) == 4 && !LIT && COLL <= LBM_COLLISION_CUM2015) {
-            if (mlp && c->cl_count % c->cl_every == 0) {
-                // network evaluated in this step; coefficients kept for the next ones
-                ma.s = a;
-                if (c->flags_needed) {
-                    if (odd) k_step_mlp<ST, COLL, true, true><<<grid, block, 0, c->stream>>>(ma);
-                    else k_step_mlp<ST, COLL, false, true><<<grid, block, 0, c->stream>>>(ma);
-                } else {
-                    if (odd) k_step_mlp<ST, COLL, true, false><<<grid, block, 0, c->stream>>>(ma);
-                    else k_step_mlp<ST, COLL, false, false><<<grid, block, 0, c->stream>>>(ma);
-                }
-            } else if (mlp) {
-                if (c->flags_needed) {
-                    if (odd) k_step<ST, COLL, false, true, true, true><<<grid, block, 0, c->stream>>>(a);
-                    else k_step<ST, COLL, false, false, true, true><<<grid, block, 0, c->stream>>>(a);
-                } else {
-                    if (odd) k_step<ST, COLL, false, true, false, true><<<grid, block, 0, c->stream>>>(a);
-                    else k_step<ST, COLL, false, false, false, true><<<grid, block, 0, c->stream>>>(a);
-                }
-            }
-            if (mlp) c->cl_count++;
-        }
-        if (!mlp) {
-            if (c->flags_needed && c->inl_deferred) {
-                if (odd) launch_flagged<ST, COLL, LIT, true, true>(grid, block, c->stream, a);
-                else launch_flagged<ST, COLL, LIT, false, true>(grid, block, c->stream, a);
-            } else if (c->flags_needed) {
-                if (odd) launch_flagged<ST, COLL, LIT, true, false>(grid, block, c->stream, a);
-                else launch_flagged<ST, COLL, LIT, false, false>(grid, block, c->stream, a);
-            } else {
-                if (odd) k_step<ST, COLL, LIT, true, false><<<grid, block, 0, c->stream>>>(a);
-                else k_step<ST, COLL, LIT, false, false><<<grid, block, 0, c->stream>>>(a);
-            }
-        }
-        HIPCHK(hipGetLastError());
-        if (patches) {
-            lbm_status st = launch_patches<ST>(c, odd ? 0 : 1);
-            if (st != LBM_OK) return st;
-        }
-        c->first = false;
-        c->steps++;
-        c->outl_pending = c->outl_deferred;
-        c->inl_pending = c->inl_deferred;
-        if (c->avg_each) {
-            c->avg_pending = true;
-            c->avg_count++;
-        }
-    }
-    HIPCHK(hipEventRecord(c->ev1, c->stream));
-    return LBM_OK;
-}
-
-template <class ST, bool LIT>
-static lbm_status launch_coll(lbm_ctx* c, int nsteps)
-{
-    switch (c->d.collision) {
-    case LBM_COLLISION_CUM2015: return launch_steps<ST, LBM_COLLISION_CUM2015, LIT>(c, nsteps);
-    case LBM_COLLISION_CUM2017: return launch_steps<ST, LBM_COLLISION_CUM2017, LIT>(c, nsteps);
-    case LBM_COLLISION_COMBINED: return launch_steps<ST, LBM_COLLISION_COMBINED, LIT>(c, nsteps);
-    default: return launch_steps<ST, LBM_COLLISION_SRT, LIT>(c, nsteps);
-    }
-}
-
-template <class ST>
-static lbm_status launch_by_coll(lbm_ctx* c, int nsteps)
-{
-    return c->d.arith == LBM_ARITH_LITERAL ? launch_coll<ST, true>(c, nsteps) : launch_coll<ST, false>(c, nsteps);
-}
-
-template <class ST>
-static lbm_status launch_by_coll_fast(lbm_ctx* c, int nsteps)
-{
-    return launch_coll<ST, false>(c, nsteps);
+    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
+    if (i < n) dst[i] = src[i];
 }
 
 // Dispatch a functor templated on the storage policy.
@@ -1157,10 +783,10 @@ lbm_status lbm_step(lbm_ctx* c, int32_t nsteps)
     switch (c->d.storage) {
     case LBM_STORAGE_F64: st = launch_by_coll<StoreF64>(c, nsteps); break;
     case LBM_STORAGE_F32: st = launch_by_coll<StoreF32>(c, nsteps); break;
-    case LBM_STORAGE_F16DEV: st = launch_by_coll_fast<StoreF16Dev>(c, nsteps); break;
-    case LBM_STORAGE_BF16DEV: st = launch_by_coll_fast<StoreBF16Dev>(c, nsteps); break;
-    case LBM_STORAGE_F16DEV_SR: st = launch_by_coll_fast<StoreF16DevSR>(c, nsteps); break;
-    case LBM_STORAGE_BF16DEV_SR: st = launch_by_coll_fast<StoreBF16DevSR>(c, nsteps); break;
+    case LBM_STORAGE_F16DEV: st = launch_by_coll<StoreF16Dev>(c, nsteps); break;
+    case LBM_STORAGE_BF16DEV: st = launch_by_coll<StoreBF16Dev>(c, nsteps); break;
+    case LBM_STORAGE_F16DEV_SR: st = launch_by_coll<StoreF16DevSR>(c, nsteps); break;
+    case LBM_STORAGE_BF16DEV_SR: st = launch_by_coll<StoreBF16DevSR>(c, nsteps); break;
     default: return LBM_E_ARG;
     }
     if (st != LBM_OK) return st;

@@ -1223,31 +1223,6 @@ __global__ __launch_bounds__(TPB) void k_error(AuxArgs<ST> a, typename ST::R* ue
     }
 }
 
-// Sum of nb per-block partial records (stride doubles apart, ncomp <= 8
-// components each) into out[0 .. ncomp), by one workgroup in a fixed order:
-// thread t adds records t, t + 256, ... in turn, then a tree over the
-// threads.  Deterministic for a given nb.
-__global__ __launch_bounds__(TPB) void k_reduce_partials(const double* parts, int nb, int stride, int ncomp,
-                                                         double* out)
-{
-    __shared__ double red[TPB][8];
-    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int b = (int)threadIdx.x; b < nb; b += TPB)
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (k < ncomp) acc[k] += parts[(size_t)b * stride + k];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) red[threadIdx.x][k] = acc[k];
-    __syncthreads();
-    for (int h = TPB / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) red[threadIdx.x][k] += red[threadIdx.x + h][k];
-        __syncthreads();
-    }
-    if ((int)threadIdx.x < ncomp) out[threadIdx.x] = red[0][threadIdx.x];
-}
-
 // Per-block FP64 sums of mass and momentum over non-solid cells.
 template <class ST>
 __global__ __launch_bounds__(TPB) void k_sums(AuxArgs<ST> a)
@@ -1389,13 +1364,6 @@ __global__ __launch_bounds__(TPB) void k_filter(AuxArgs<ST> a, int fct, int cx, 
     const double inv = cnt ? 1.0 / cnt : 0.0;
 #pragma unroll
     for (int k = 0; k < 10; ++k) a.io[k * NC + ic] = acc[k] * inv;
-}
-
-// Plain stream copy used as the bandwidth reference.
-__global__ __launch_bounds__(TPB) void k_copy(const float4* __restrict__ src, float4* __restrict__ dst, size_t n)
-{
-    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
-    if (i < n) dst[i] = src[i];
 }
 
 }  // namespace lbm
