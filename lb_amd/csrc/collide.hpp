@@ -89,6 +89,55 @@ LBM_HD R frcp(R x)
     return R(1) / x;
 }
 
+template <class R>
+LBM_HD R fma_r(R a, R b, R c)
+{
+    return std::fma(a, b, c);
+}
+
+// Reciprocal of a positive normal number (a density, a relaxation time): the
+// hardware FP32 reciprocal and one Newton step in fused multiply-adds, which
+// leave the error at the half ulp of the last rounding, in 3 instructions
+// where the IEEE quotient's scaling and fix-up take 11.
+template <class R>
+LBM_HD R rcp_nr(R x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (sizeof(R) == 4) {
+        const R r = __builtin_amdgcn_rcpf(x);
+        return fma_r(fma_r(-x, r, R(1)), r, r);
+    }
+#endif
+    return R(1) / x;
+}
+
+// Square root of a positive normal number: the hardware inverse square root
+// and one correction, exact to the half ulp of the last rounding (5
+// instructions; the IEEE square root takes 16).
+template <class R>
+LBM_HD R sqrt_nr(R x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (sizeof(R) == 4) {
+        const R y = __builtin_amdgcn_rsqf(x);
+        const R s = x * y;
+        return fma_r(fma_r(-s, s, x), R(0.5) * y, s);
+    }
+#endif
+    return std::sqrt(x);
+}
+
+// Square root, 0 included: the hardware FP32 instruction (within 1 ulp) on
+// the device, correctly rounded otherwise.
+template <class R>
+LBM_HD R fsqrt(R x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (sizeof(R) == 4) return __builtin_amdgcn_sqrtf(x);
+#endif
+    return std::sqrt(x);
+}
+
 // Base-10 logarithm for the closure features: the hardware log2 (within
 // 1 ulp for normal inputs) times log10(2) on the device in FP32, the library
 // function otherwise.
@@ -775,6 +824,410 @@ LBM_HD void cum2017_fast(const Consts<R>& K, const R* fin, const Cen2<R>& c, R m
 #pragma unroll
     for (int q = 0; q < Q; ++q) f[q] = X[CELL3(q)];
 }
+
+// ---------------------------------------------------------------------------
+// The same operators in fewer operations, for the storage formats whose
+// results may be rounded differently (see Ops below).
+// ---------------------------------------------------------------------------
+
+// Sum (x - ux)^2 f = mxx - ux (jx + k100) and sum (x - ux)(y - uy) f =
+// mxy - ux jy - uy k100, with k100 = jx - ux m0 (rounding-small, except on
+// the first step after an initialisation): 15 multiply-adds and three sums
+// where the written-out squares take 57 operations, and fewer roundings.
+// Fused multiply-adds are written out and contraction is off, here and in the
+// functions below: every kernel that forms the rate gets the same bits.
+template <class R>
+LBM_HD Cen2<R> central2_fused(const Raw2<R>& r, R ux, R uy, R uz)
+{
+    LBM_FP_STRICT
+    Cen2<R> c;
+    c.k100 = fma_r(-ux, r.m0, r.jx);
+    c.k010 = fma_r(-uy, r.m0, r.jy);
+    c.k001 = fma_r(-uz, r.m0, r.jz);
+    c.kxx = fma_r(-ux, r.jx + c.k100, r.mxx);
+    c.kyy = fma_r(-uy, r.jy + c.k010, r.myy);
+    c.kzz = fma_r(-uz, r.jz + c.k001, r.mzz);
+    c.kxy = fma_r(-uy, c.k100, fma_r(-ux, r.jy, r.mxy));
+    c.kxz = fma_r(-uz, c.k100, fma_r(-ux, r.jz, r.mxz));
+    c.kyz = fma_r(-uz, c.k010, fma_r(-uy, r.jz, r.myz));
+    return c;
+}
+
+// |Pi_neq| / rho: see omega_les_fast.  For D3Q27 the second-order equilibrium moments are
+// rho*(u u + I/3), so Pi_neq = central second moments - rho/3 I (the
+// reference builds the same tensor with a 27-term loop, OmegaLES.h:84-101).
+// The norm's argument carries the cancellation error of that difference
+// (about 1e-3 relative in FP32), so the hardware square root (within 1 ulp)
+// adds nothing to it.
+template <class R>
+LBM_HD R pin_over_rho_fused(const Cen2<R>& c, R rho)
+{
+    LBM_FP_STRICT
+    const R pxx = fma_r(R(-1.0 / 3.0), rho, c.kxx), pyy = fma_r(R(-1.0 / 3.0), rho, c.kyy),
+            pzz = fma_r(R(-1.0 / 3.0), rho, c.kzz);
+    const R off = fma_r(c.kxy, c.kxy, fma_r(c.kxz, c.kxz, c.kyz * c.kyz));
+    const R n2 = fma_r(R(2), off, fma_r(pxx, pxx, fma_r(pyy, pyy, pzz * pzz)));
+    return fsqrt(n2) * rcp_nr(rho);
+}
+
+// Relaxation time from a coefficient C: the reference's formula
+// tau/2 + sqrt(tau^2 + 18 C |Pi_neq| / rho) / 2 (OmegaLES.h:103-131).
+template <class R>
+LBM_HD R tau_from_coefficient_fused(R C, R pin_rho, R tau0)
+{
+    LBM_FP_STRICT
+    return fma_r(R(0.5), sqrt_nr(fma_r(R(18) * C, pin_rho, tau0 * tau0)), R(0.5) * tau0);
+}
+
+// Rate from a closure coefficient C.
+template <class R>
+LBM_HD R omega_from_coefficient_fused(R C, R pin_rho, R tau0)
+{
+    return rcp_nr(tau_from_coefficient_fused(C, pin_rho, tau0));
+}
+
+// Smagorinsky rate from the non-equilibrium stress; the learned closure's
+// fallback evaluates this same formula in another kernel.
+template <class R>
+LBM_HD R omega_les_fused(const Cen2<R>& c, R rho, R tau, R cles)
+{
+    return omega_from_coefficient_fused(cles, pin_over_rho_fused(c, rho), tau);
+}
+
+// Inverse line transform along one axis: central moments (a0, a1, a2) about u
+// to populations at c = -1, 0, +1.  With S = a0 u^2 + 2 u a1 + a2 and
+// D = a0 u + a1 these are (S - D)/2, a0 - S, (S + D)/2.  The moments come
+// scaled, a1/2 and a2/2 (every moment of the transform carries a factor 1/2
+// per axis along which its order is not 0), so that no halving is left:
+// 6 operations a line instead of 8.
+template <class R>
+struct LineU {
+    R u2, uh, uuh;   // 2 u, u/2, u^2/2
+    LBM_HD explicit LineU(R u) : u2(R(2) * u), uh(R(0.5) * u), uuh(R(0.5) * u * u) {}
+};
+
+template <class R>
+LBM_HD void inv_line(R a0, R a1h, R a2h, const LineU<R>& l, R& fm, R& fz, R& fp)
+{
+    LBM_FP_STRICT
+    const R S = fma_r(a0, l.uuh, fma_r(l.u2, a1h, a2h)), D = fma_r(a0, l.uh, a1h);
+    fm = S - D;
+    fz = fma_r(R(-2), S, a0);
+    fp = S + D;
+}
+
+// The same with a1 = 0, with a2 = 0, and with a1 alone.
+template <class R>
+LBM_HD void inv_line_02(R a0, R a2h, const LineU<R>& l, R& fm, R& fz, R& fp)
+{
+    LBM_FP_STRICT
+    const R S = fma_r(a0, l.uuh, a2h), D = a0 * l.uh;
+    fm = S - D;
+    fz = fma_r(R(-2), S, a0);
+    fp = S + D;
+}
+
+template <class R>
+LBM_HD void inv_line_01(R a0, R a1h, const LineU<R>& l, R& fm, R& fz, R& fp)
+{
+    LBM_FP_STRICT
+    const R S = fma_r(a0, l.uuh, l.u2 * a1h), D = fma_r(a0, l.uh, a1h);
+    fm = S - D;
+    fz = fma_r(R(-2), S, a0);
+    fp = S + D;
+}
+
+template <class R>
+LBM_HD void inv_line_1(R a1h, const LineU<R>& l, R& fm, R& fz, R& fp)
+{
+    LBM_FP_STRICT
+    const R S = l.u2 * a1h;
+    fm = S - a1h;
+    fz = R(-2) * S;
+    fp = S + a1h;
+}
+
+// y and z passes of the inverse transform: X[9 a + 3 oy + oz] (a the x class,
+// oy and oz the orders still to be transformed, scaled) to populations.
+template <class R>
+LBM_HD void inv_yz(R* X, R uy, R uz, R* f)
+{
+    const LineU<R> ly(uy), lz(uz);
+    R Y[27];   // Y[9*a + 3*b + oz]
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int oz = 0; oz < 3; ++oz)
+            inv_line(X[9 * a + oz], X[9 * a + 3 + oz], X[9 * a + 6 + oz], ly, Y[9 * a + oz], Y[9 * a + 3 + oz],
+                     Y[9 * a + 6 + oz]);
+#pragma unroll
+    for (int ab = 0; ab < 9; ++ab)
+        inv_line(Y[3 * ab], Y[3 * ab + 1], Y[3 * ab + 2], lz, X[3 * ab], X[3 * ab + 1], X[3 * ab + 2]);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) f[q] = X[CELL3(q)];
+}
+
+// Reduced cumulant collision.  m0 is the zeroth moment of f, rho/u the
+// fields the step uses (equal to the moments of f except on the first step
+// after an equilibrium initialisation).  Writes post-collision populations.
+//
+// What bounds it is the number of vector instructions: 16-bit storage moves
+// so few bytes that the step waits for them, and FP32 does once two steps
+// share one pass over memory.  With every cumulant of order >= 3 zero the
+// state is a Gaussian, whose moments of order 4 and 6 follow from those of
+// order 2 (Eq. G2015 81-84 with those cumulants dropped): in
+// x = s200, ..., over rho, s220 = rho (ab + 2 d^2), s211 = rho (a f + 2 d e)
+// and s222 = i200 s022 + 2 i110 s112 + 2 i101 s121, three multiply-adds where
+// the written-out Eq. 84 takes 28 operations.  The moments are formed with the
+// factor 2^-(axes of non-zero order) that inv_line wants (h: 1/2, q: 1/4,
+// e: 1/8; the factors are powers of two and cost nothing).
+template <class R>
+LBM_HD void cum2015_fused(const Consts<R>& K, const Cen2<R>& c, R m0, R rho, R ux, R uy, R uz, R omg, R* f)
+{
+    LBM_FP_STRICT
+    const R ir = rcp_nr(rho);
+    const R C200 = c.kxx, C020 = c.kyy, C002 = c.kzz;
+    const R d1 = C200 - C020, d2 = C200 - C002;
+    const R hw = R(0.5) * omg * ir, hw3 = R(3) * hw;
+    const R Dxu = -fma_r(hw, d1 + d2, R(0.5) * ir * (C200 + C020 + C002 - m0));
+    const R Dyv = fma_r(hw3, d1, Dxu), Dzw = fma_r(hw3, d2, Dxu);
+    const R om1 = R(1) - omg;
+    const R A = rho * fma_r(R(-1.5), omg, R(3));
+    const R xx = ux * ux * Dxu, yy = uy * uy * Dyv, zz = uz * uz * Dzw;
+    const R e61 = fma_r(om1, d1, -A * (xx - yy));
+    const R e64 = fma_r(om1, d2, -A * (xx - zz));
+    const R e65 = fma_r(R(-1.5) * rho, xx + yy + zz, m0);
+    const R c13h = R(0.5) * K.c13;
+    const R s200h = c13h * (e61 + e64 + e65);
+    const R s020h = c13h * fma_r(R(-2), e61, e64 + e65);
+    const R s002h = c13h * fma_r(R(-2), e64, e61 + e65);
+    const R om1q = R(0.25) * om1;
+    const R s110q = om1q * c.kxy, s101q = om1q * c.kxz, s011q = om1q * c.kyz;
+    // order-4 and order-6 central moments of the post-collision state
+    const R i200h = s200h * ir, i020h = s020h * ir, i002h = s002h * ir;
+    const R i110q = s110q * ir, i101q = s101q * ir, i011q = s011q * ir;
+    const R g110 = R(4) * i110q, g101 = R(4) * i101q, g011 = R(4) * i011q;
+    const R s211e = fma_r(s200h, i011q, s101q * g110);
+    const R s121e = fma_r(s020h, i101q, s110q * g011);
+    const R s112e = fma_r(s002h, i110q, s011q * g101);
+    const R s220q = fma_r(s020h, i200h, R(2) * s110q * g110);
+    const R s022q = fma_r(s002h, i020h, R(2) * s011q * g011);
+    const R s202q = fma_r(s200h, i002h, R(2) * s101q * g101);
+    const R s222e = fma_r(i200h, s022q, R(2) * fma_r(g110, s112e, g101 * s121e));
+
+    // x pass: (order_x 0,1,2) -> (m, z, p) for each (order_y, order_z)
+    const LineU<R> lx(ux);
+    R X[27];  // X[9*a + 3*oy + oz], a = x class
+#define XL(oy, oz) X[3 * (oy) + (oz)], X[9 + 3 * (oy) + (oz)], X[18 + 3 * (oy) + (oz)]
+    inv_line(m0, R(-0.5) * c.k100, s200h, lx, XL(0, 0));
+    inv_line_01(R(-0.5) * c.k001, s101q, lx, XL(0, 1));
+    inv_line_02(s002h, s202q, lx, XL(0, 2));
+    inv_line_01(R(-0.5) * c.k010, s110q, lx, XL(1, 0));
+    inv_line_02(s011q, s211e, lx, XL(1, 1));
+    inv_line_1(s112e, lx, XL(1, 2));
+    inv_line_02(s020h, s220q, lx, XL(2, 0));
+    inv_line_1(s121e, lx, XL(2, 1));
+    inv_line_02(s022q, s222e, lx, XL(2, 2));
+#undef XL
+    inv_yz(X, uy, uz, f);
+}
+
+// Raw moments of order 3 that the 2017 operator relaxes.
+template <class R>
+struct Raw3 {
+    R m120, m102, m210, m012, m201, m021, m111;
+};
+
+template <class R>
+LBM_HD Raw3<R> raw3(const R* f)
+{
+    // sums over z of each (cx, cy) line, as in raw_moments (the compiler
+    // shares them)
+    R s0[9], s1[9], s2[9];
+#pragma unroll
+    for (int ab = 0; ab < 9; ++ab) {
+        R m = R(0), z = R(0), p = R(0);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            if (3 * (CX[q] + 1) + (CY[q] + 1) != ab) continue;
+            if (CZ[q] < 0) m = f[q];
+            else if (CZ[q] == 0) z = f[q];
+            else p = f[q];
+        }
+        s2[ab] = p + m;
+        s1[ab] = p - m;
+        s0[ab] = s2[ab] + z;
+    }
+    R t10[3], t20[3], t01[3], t02[3], t11[3], t21[3], t12[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int m = 3 * a, z = 3 * a + 1, p = 3 * a + 2;
+        t20[a] = s0[p] + s0[m];
+        t10[a] = s0[p] - s0[m];
+        t11[a] = s1[p] - s1[m];
+        t21[a] = s1[p] + s1[m];
+        t12[a] = s2[p] - s2[m];
+        t01[a] = t21[a] + s1[z];
+        t02[a] = s2[p] + s2[m] + s2[z];
+    }
+    Raw3<R> r;
+    r.m120 = t20[2] - t20[0];
+    r.m102 = t02[2] - t02[0];
+    r.m210 = t10[2] + t10[0];
+    r.m201 = t01[2] + t01[0];
+    r.m012 = t12[2] + t12[0] + t12[1];
+    r.m021 = t21[2] + t21[0] + t21[1];
+    r.m111 = t11[2] - t11[0];
+    return r;
+}
+
+template <int V, class R>
+LBM_HD void cum2017_fused(const Consts<R>& K, const R* fin, const Cen2<R>& c, R m0, R rho, R ux, R uy, R uz, R omg,
+                         R* f)
+{
+    const Raw2<R> r = raw_moments(fin);
+    const Raw3<R> t = raw3(fin);
+    // central third moments from the raw ones: with y' = y - uy,
+    // sum (x - ux) y'^2 f = m120 - ux myy - uy (2 kxy + uy k100), and so on
+    auto third = [](R m, R u, R mvv, R v, R kuv, R ku) {
+        LBM_FP_STRICT
+        return fma_r(-v, fma_r(v, ku, R(2) * kuv), fma_r(-u, mvv, m));
+    };
+    const R C120 = third(t.m120, ux, r.myy, uy, c.kxy, c.k100), C102 = third(t.m102, ux, r.mzz, uz, c.kxz, c.k100);
+    const R C210 = third(t.m210, uy, r.mxx, ux, c.kxy, c.k010), C012 = third(t.m012, uy, r.mzz, uz, c.kyz, c.k010);
+    const R C201 = third(t.m201, uz, r.mxx, ux, c.kxz, c.k001), C021 = third(t.m021, uz, r.myy, uy, c.kyz, c.k001);
+    const R C111 = fma_r(-ux, c.kyz, fma_r(-uy, fma_r(-uz, r.jx, r.mxz), fma_r(-uz, r.mxy, t.m111)));
+    const R ir = rcp_nr(rho);
+    const R C200 = c.kxx, C020 = c.kyy, C002 = c.kzz;
+
+    // rates and limiters (Turbulent2017.h:240-291) with omega_2 = 1 substituted
+    const R w1 = omg;
+    const R w3 = -R(8) * (w1 - R(2)) * (R(2) * w1 + R(1)) * frcp(R(8) + w1 * (R(14) - R(7) * w1));
+    const R w4 = R(8) * (w1 - R(2)) * (R(4) * w1 - R(7)) * frcp(R(56) - R(50) * w1 + K.w4q * w1 * w1);
+    const R w5 = R(24) * (w1 - R(2)) * (R(2) + w1 * (R(7) - R(3) * w1)) *
+                 frcp(R(16) * w1 * w1 * (w1 - R(6)) - R(2) * w1 * (R(216) + R(5) * w1 * (R(9) * w1 - R(46))) +
+                      (w1 * (R(3) * w1 - R(10)) * (R(15) * w1 - R(28)) - R(48)));
+    const R iden = frcp((w1 - R(1)) * (R(2) - R(5) * w1));
+    const R A = (R(4) * w1 * w1 + R(2) * w1 * (w1 - R(6)) + w1 * (R(10) - R(3) * w1) - R(4)) * iden;
+    const R B = (R(4) * w1 * (R(9) * w1 - R(16)) - R(4) * w1 * w1 - R(2) * (R(2) + R(9) * w1 * (w1 - R(2)))) *
+                (iden * R(1.0 / 3.0));
+    const R rl = rho * K.lam;
+    auto lim = [rl](R w, R a) {
+        const R m = std::fabs(a);
+        return (R(1) - w) * rl * frcp(rl + m);   // 1 - (w + (1 - w) |a| / (rl + |a|))
+    };
+    const R p120 = C120 + C102, m120 = C120 - C102;
+    const R p210 = C210 + C012, m210 = C210 - C012;
+    const R p201 = C201 + C021, m201 = C201 - C021;
+    const R e117 = lim(w3, p120) * p120;
+    const R e118 = lim(w3, K.lim210 ? p120 : p210) * p210;
+    const R e119 = lim(w3, p201) * p201;
+    const R e120 = lim(w4, m120) * m120;
+    const R e121 = lim(w4, K.lim210 ? m120 : m210) * m210;
+    const R e122 = lim(w4, m201) * m201;
+    const R s120 = R(0.5) * (e120 + e117), s102 = R(0.5) * (e117 - e120);
+    const R s210 = R(0.5) * (e121 + e118), s012 = R(0.5) * (e118 - e121);
+    const R s201 = R(0.5) * (e122 + e119), s021 = R(0.5) * (e119 - e122);
+    const R s111 = lim(w5, C111) * C111;
+
+    // second order as in the 2015 operator, with the 2017 bulk term
+    R tr = m0;
+    if (K.trace17) tr = V == CV_2017 ? rho - R(1) : rho + R(1);
+    const R hw = R(0.5) * omg * ir;
+    const R Dxu = -hw * (R(2) * C200 - C020 - C002) - R(0.5) * ir * (C200 + C020 + C002 - tr);
+    const R Dyv = Dxu + R(3) * hw * (C200 - C020);
+    const R Dzw = Dxu + R(3) * hw * (C200 - C002);
+    const R om1 = R(1) - omg;
+    const R A3 = R(3) * rho * (R(1) - R(0.5) * omg);
+    const R xx = ux * ux * Dxu, yy = uy * uy * Dyv, zz = uz * uz * Dzw;
+    const R e61 = om1 * (C200 - C020) - A3 * (xx - yy);
+    const R e64 = om1 * (C200 - C002) - A3 * (xx - zz);
+    const R e65 = m0 - R(1.5) * rho * (xx + yy + zz);
+    const R s200 = K.c13 * (e61 + e64 + e65);
+    const R s020 = K.c13 * (e64 - R(2) * e61 + e65);
+    const R s002 = K.c13 * (e61 - R(2) * e64 + e65);
+    const R s110 = om1 * c.kxy, s101 = om1 * c.kxz, s011 = om1 * c.kyz;
+
+    // fourth-order cumulants, Eq. G2017 43-48 with omega_6..8 = 1: (1/omega_1 - 1/2) rho A, B
+    const R g = (frcp(w1) - R(0.5)) * rho;
+    const R ga = g * A, gb = -K.c13 * g * B * (-R(3) * w1 * ir);
+    const R e43 = K.c23 * ga * (Dxu - R(2) * Dyv + Dzw);
+    const R e44 = K.c23 * ga * (K.eq44 ? (Dxu + Dyv - R(2) * Dzw) : (Dyv + Dzw - R(2) * Dxu));
+    const R e45 = -K.c43 * ga * (Dxu + Dyv + Dzw);
+    const R c220 = K.c13 * (e43 + e44 + e45), c202 = K.c13 * (e45 - e43), c022 = K.c13 * (e45 - e44);
+    const R c211 = gb * c.kyz, c121 = gb * c.kxz, c112 = gb * c.kxy;
+
+    // back to central moments, Eq. G2015 81-84 (orders 5 and 6 from products)
+    R s[27];
+#define S_(i, j, l) s[9 * (i) + 3 * (j) + (l)]
+    S_(0, 0, 0) = m0;
+    S_(1, 0, 0) = -c.k100;
+    S_(0, 1, 0) = -c.k010;
+    S_(0, 0, 1) = -c.k001;
+    S_(2, 0, 0) = s200, S_(0, 2, 0) = s020, S_(0, 0, 2) = s002;
+    S_(1, 1, 0) = s110, S_(1, 0, 1) = s101, S_(0, 1, 1) = s011;
+    S_(1, 2, 0) = s120, S_(1, 0, 2) = s102, S_(2, 1, 0) = s210;
+    S_(0, 1, 2) = s012, S_(2, 0, 1) = s201, S_(0, 2, 1) = s021, S_(1, 1, 1) = s111;
+    S_(2, 1, 1) = c211 + (s200 * s011 + R(2) * s101 * s110) * ir;
+    S_(1, 2, 1) = c121 + (s020 * s101 + R(2) * s110 * s011) * ir;
+    S_(1, 1, 2) = c112 + (s002 * s110 + R(2) * s011 * s101) * ir;
+    S_(2, 2, 0) = c220 + (s020 * s200 + R(2) * s110 * s110) * ir;
+    S_(0, 2, 2) = c022 + (s002 * s020 + R(2) * s011 * s011) * ir;
+    S_(2, 0, 2) = c202 + (s200 * s002 + R(2) * s101 * s101) * ir;
+    S_(1, 2, 2) = (s020 * s102 + s002 * s120 + R(4) * s011 * s111 + R(2) * (s110 * s012 + s101 * s021)) * ir;
+    S_(2, 1, 2) = (s002 * s210 + s200 * s012 + R(4) * s101 * s111 + R(2) * (s011 * s201 + s110 * s102)) * ir;
+    S_(2, 2, 1) = (s200 * s021 + s020 * s201 + R(4) * s110 * s111 + R(2) * (s101 * s120 + s011 * s210)) * ir;
+    S_(2, 2, 2) = (R(4) * s111 * s111 + s200 * S_(0, 2, 2) + s020 * S_(2, 0, 2) + s002 * S_(2, 2, 0) +
+                   R(4) * (s011 * S_(2, 1, 1) + s101 * S_(1, 2, 1) + s110 * S_(1, 1, 2)) +
+                   R(2) * (s120 * s102 + s210 * s012 + s201 * s021)) * ir -
+                  (R(16) * s110 * s101 * s011 + R(4) * (s101 * s101 * s020 + s011 * s011 * s200 + s110 * s110 * s002) +
+                   R(2) * s200 * s020 * s002) * ir * ir;
+#undef S_
+    // x, y, z passes of the backward transform, on moments scaled as inv_line
+    // wants them
+#pragma unroll
+    for (int i = 1; i < 27; ++i)
+        s[i] *= R(1) / R(1 << ((i / 9 != 0) + (i / 3 % 3 != 0) + (i % 3 != 0)));
+    const LineU<R> lx(ux);
+    R X[27];
+#pragma unroll
+    for (int bc = 0; bc < 9; ++bc) inv_line(s[bc], s[9 + bc], s[18 + bc], lx, X[bc], X[9 + bc], X[18 + bc]);
+    inv_yz(X, uy, uz, f);
+}
+
+// Which of the two forms a kernel runs.  FP32 storage keeps the written-out
+// operation order: its results are compared with earlier ones at single
+// precision, and a uniform stream rounds alike in every cell, so that another
+// order drifts away from it by 1e-4 of a cross-stream velocity in 300 steps.
+// For 16-bit storage such differences vanish in the rounding of the stored
+// populations, and in FP64 they are 1e-15.
+template <bool FUSED>
+struct Ops {
+    template <class R>
+    LBM_HD static R rcp(R x)
+    {
+        if constexpr (FUSED) return rcp_nr(x);
+        return R(1) / x;
+    }
+    template <class R>
+    LBM_HD static Cen2<R> cen2(const Raw2<R>& r, R ux, R uy, R uz)
+    {
+        if constexpr (FUSED) return central2_fused(r, ux, uy, uz);
+        return central2(r, ux, uy, uz);
+    }
+    template <class R>
+    LBM_HD static R omega_les(const Cen2<R>& c, R rho, R tau, R cles)
+    {
+        if constexpr (FUSED) return omega_les_fused(c, rho, tau, cles);
+        return omega_les_fast(c, rho, tau, cles);
+    }
+    template <class R>
+    LBM_HD static void cum2015(const Consts<R>& K, const Cen2<R>& c, R m0, R rho, R ux, R uy, R uz, R omg, R* f)
+    {
+        if constexpr (FUSED) cum2015_fused(K, c, m0, rho, ux, uy, uz, omg, f);
+        else cum2015_fast(K, c, m0, rho, ux, uy, uz, omg, f);
+    }
+};
 
 // BGK with the closed-form equilibrium (fast variant).
 template <class R>

@@ -431,12 +431,6 @@ __device__ __forceinline__ void inlet_rule(const Consts<R>& K, const NodeDev& b,
         zou_he(K, b, crev20, post, own[0], own[1], own[2], own[3], st);
 }
 
-template <class R>
-__device__ __forceinline__ R fast_rcp(R x)
-{
-    return R(1) / x;
-}
-
 // Caller-layout index of a padded cell.
 __device__ __forceinline__ size_t user_index(const Geo& g, const Cell& c)
 {
@@ -579,6 +573,7 @@ __device__ __forceinline__ void closure_prep(const typename ST::R* f, bool first
                                              const MlpLds& L, ClosurePrep<ST>& o)
 {
     using R = typename ST::R;
+    using O = Ops<ST::fused>;
     const Raw2<R> r = raw_moments(f);
     o.m0 = r.m0;
     if (first) {
@@ -588,13 +583,13 @@ __device__ __forceinline__ void closure_prep(const typename ST::R* f, bool first
         o.uz = macro[3 * N + i];
     } else {
         o.rho = r.m0;
-        const R ir = fast_rcp(o.rho);
+        const R ir = O::rcp(o.rho);
         o.ux = r.jx * ir;
         o.uy = r.jy * ir;
         o.uz = r.jz * ir;
     }
-    o.ce = central2(r, o.ux, o.uy, o.uz);
-    o.om_s = omega_les_fast(o.ce, o.rho, tau, cles);
+    o.ce = O::cen2(r, o.ux, o.uy, o.uz);
+    o.om_s = O::omega_les(o.ce, o.rho, tau, cles);
     R om_unused;
     cell_features(o.ce, o.rho, tau, cles, o.x, o.pin, om_unused);
     o.env = mlp_normalise(L, o.x, o.xn);
@@ -649,7 +644,7 @@ __global__ __launch_bounds__(TPB) void k_step_mlp(MlpStepArgs<ST> ma)
         if (a.ccache) a.ccache[c.i] = cp.env ? mlp_coefficient(z, ma.mlp.c) : (float)a.cles;
         R P[Q];
         if (COLL == LBM_COLLISION_CUM2015) {
-            cum2015_fast(a.K, cp.ce, cp.m0, cp.rho, cp.ux, cp.uy, cp.uz, omega, P);
+            Ops<ST::fused>::cum2015(a.K, cp.ce, cp.m0, cp.rho, cp.ux, cp.uy, cp.uz, omega, P);
         } else {
 #pragma unroll
             for (int q = 0; q < Q; ++q) P[q] = f[q];
@@ -1095,16 +1090,17 @@ __device__ __forceinline__ void cell_macro(const AuxArgs<ST>& a, const Cell& c, 
             uz = r.jz / rho;
         }
         if (om) {
+            using O = Ops<ST::fused>;
             // the rate from the velocity as the step forms it (reciprocal, then products)
             R vx = ux, vy = uy, vz = uz;
             if (!a.first) {
-                const R ir = fast_rcp(rho);
+                const R ir = O::rcp(rho);
                 vx = r.jx * ir;
                 vy = r.jy * ir;
                 vz = r.jz * ir;
             }
-            const Cen2<R> ce = central2(r, vx, vy, vz);
-            *om = sponge(a.closure == LBM_CLOSURE_SMAGORINSKY ? omega_les_fast(ce, rho, a.tau, a.cles) : a.omega0,
+            const Cen2<R> ce = O::cen2(r, vx, vy, vz);
+            *om = sponge(a.closure == LBM_CLOSURE_SMAGORINSKY ? O::omega_les(ce, rho, a.tau, a.cles) : a.omega0,
                          a.sp_axis, a.sp_begin, a.sp_deriv, a.g, c.x, c.y, c.z);
         }
     }

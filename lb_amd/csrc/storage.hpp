@@ -9,7 +9,8 @@
 // the *SR policies and to nearest in the others, and takes the streaming
 // hint NT; the collide-stream kernel uses it for the populations it streams,
 // all other writers use the first form.  load(p, i, rest) and
-// get<NT>(p, i, rest) likewise.
+// get<NT>(p, i, rest) likewise.  `fused` picks the form of the fast arithmetic
+// (collide.hpp, Ops).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -59,6 +60,7 @@ struct StoreF64 {
     using T = double;   // element in HBM
     using R = double;   // arithmetic type
     static constexpr bool dev = false;
+    static constexpr bool fused = true;
     static constexpr bool sr = false;
     // the value a store then a load would return
     __device__ __forceinline__ static R round_trip(R v, R) { return v; }
@@ -80,6 +82,7 @@ struct StoreF32 {
     using T = float;
     using R = float;
     static constexpr bool dev = false;
+    static constexpr bool fused = false;
     static constexpr bool sr = false;
     __device__ __forceinline__ static R round_trip(R v, R) { return v; }
     __device__ __forceinline__ static R load(const T* p, uint32_t i, R) { return at(p, i); }
@@ -100,6 +103,7 @@ struct StoreF16Dev {
     using T = _Float16;
     using R = float;
     static constexpr bool dev = true;
+    static constexpr bool fused = true;
     static constexpr bool sr = false;
     __device__ __forceinline__ static R load(const T* p, uint32_t i, R rest) { return (float)at(p, i) + rest; }
     __device__ __forceinline__ static void store(T* p, uint32_t i, R v, R rest) { at(p, i) = (_Float16)(v - rest); }
@@ -121,6 +125,7 @@ struct StoreBF16Dev {
     using T = uint16_t;
     using R = float;
     static constexpr bool dev = true;
+    static constexpr bool fused = true;
     static constexpr bool sr = false;
     __device__ __forceinline__ static R load(const T* p, uint32_t i, R rest)
     {
