@@ -41,11 +41,29 @@ struct GradArgs {
     double* part_loss;    // [gridDim.x]
 };
 
-struct TrainLds {
+// Weights and staging of one training workgroup.  For the matrix cores the
+// weights sit in fragment order as BF16, rounded once per workgroup: entry
+// [..][lane] is what that lane feeds the instruction, so a fragment is 64
+// consecutive 8-byte words.  (Read as FP32 rows and rounded at every use they
+// cost a 16-way bank conflict and 16 vector instructions each, 36 times a tile.)
+template <bool BF>
+struct TrainWeights {
     float w1[NHID * 16];
     float w2[NHID * NHID];
-    float b1[NHID], b2[NHID], w3[NHID];
     float ea[4][256], eb[4][256];
+};
+
+template <>
+struct TrainWeights<true> {
+    bf16x4 w1f[4][64];       // [hidden block][lane]: W1[16 hb + s][4 q ..]
+    bf16x4 w2f[4][4][64];    // [out block][in block][lane]: W2[16 mb + s][16 kb + 4 q ..]
+    bf16x4 w2t[4][4][64];    // [in block][out block][lane]: W2[16 kb + 4 q ..][16 hb + s]
+};
+
+template <bool BF>
+struct TrainLds {
+    TrainWeights<BF> w;
+    float b1[NHID], b2[NHID], w3[NHID];
     union {
         struct {
             float t1[4][NHID * 16];
@@ -70,22 +88,35 @@ __device__ __forceinline__ int64_t sample_index(const GradArgs& a, int64_t pos)
     return (int64_t)(h % (uint64_t)a.n);
 }
 
+// Operand fragment of a product: four FP32 values, or their BF16 roundings.
+template <bool BF>
+struct FragOf {
+    using T = f32x4;
+};
+template <>
+struct FragOf<true> {
+    using T = bf16x4;
+};
+template <bool BF>
+using Frag = typename FragOf<BF>::T;
+
+template <bool BF>
+__device__ __forceinline__ Frag<BF> frag(f32x4 v)
+{
+    if constexpr (BF) return pack_bf16x4(v[0], v[1], v[2], v[3]);
+    else return v;
+}
+
 // D = A B + C for one 16x16x16 tile (fragments in the mlp.hpp layout).
 template <bool BF>
-__device__ __forceinline__ f32x4 mma(TrainLds& L, int wave, f32x4 a, f32x4 b, f32x4 c)
+__device__ __forceinline__ f32x4 mma(TrainLds<BF>& L, int wave, Frag<BF> a, Frag<BF> b, f32x4 c)
 {
     if constexpr (BF) {
-        bf16x4 ab, bb;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            ab[j] = f2bf(a[j]);
-            bb[j] = f2bf(b[j]);
-        }
-        return mfma_bf16(ab, bb, c);
+        return mfma_bf16(a, b, c);
     } else {
         const int lane = threadIdx.x & 63, q = lane >> 4, s = lane & 15;
-        float* EA = L.ea[wave];
-        float* EB = L.eb[wave];
+        float* EA = L.w.ea[wave];
+        float* EB = L.w.eb[wave];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             EA[s * 16 + 4 * q + j] = a[j];
@@ -106,21 +137,79 @@ __device__ __forceinline__ f32x4 mma(TrainLds& L, int wave, f32x4 a, f32x4 b, f3
     }
 }
 
+// Weight fragments: W1 block hb; W2 rows of block mb, columns of block kb; and
+// its transpose.
+template <bool BF>
+__device__ __forceinline__ Frag<BF> w1_frag(const TrainLds<BF>& L, int hb)
+{
+    const int lane = threadIdx.x & 63, q = lane >> 4, s = lane & 15;
+    if constexpr (BF) return L.w.w1f[hb][lane];
+    else return *(const f32x4*)&L.w.w1[(hb * 16 + s) * 16 + 4 * q];
+}
+template <bool BF>
+__device__ __forceinline__ Frag<BF> w2_frag(const TrainLds<BF>& L, int mb, int kb)
+{
+    const int lane = threadIdx.x & 63, q = lane >> 4, s = lane & 15;
+    if constexpr (BF) return L.w.w2f[mb][kb][lane];
+    else return *(const f32x4*)&L.w.w2[(mb * 16 + s) * NHID + kb * 16 + 4 * q];
+}
+template <bool BF>
+__device__ __forceinline__ Frag<BF> w2t_frag(const TrainLds<BF>& L, int hb, int kb)
+{
+    const int lane = threadIdx.x & 63, q = lane >> 4, s = lane & 15;
+    if constexpr (BF) {
+        return L.w.w2t[hb][kb][lane];
+    } else {
+        f32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = L.w.w2[(kb * 16 + 4 * q + j) * NHID + hb * 16 + s];
+        return w;
+    }
+}
+
+template <bool BF>
+__device__ __forceinline__ void load_weights(TrainLds<BF>& L, const float* p)
+{
+    const int tid = threadIdx.x;
+    if constexpr (BF) {
+        const int lane = tid & 63, q = lane >> 4, s = lane & 15, wv = tid >> 6;
+        {
+            f32x4 v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = 4 * q + j < NFEAT ? p[OFF_W1 + (wv * 16 + s) * NFEAT + 4 * q + j] : 0.0f;
+            L.w.w1f[wv][lane] = frag<BF>(v);
+        }
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            f32x4 v, t;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] = p[OFF_W2 + (wv * 16 + s) * NHID + kb * 16 + 4 * q + j];
+                t[j] = p[OFF_W2 + (kb * 16 + 4 * q + j) * NHID + wv * 16 + s];
+            }
+            L.w.w2f[wv][kb][lane] = frag<BF>(v);
+            L.w.w2t[wv][kb][lane] = frag<BF>(t);
+        }
+    } else {
+        for (int i = tid; i < NHID * 16; i += TPB_T) {
+            const int h = i >> 4, k = i & 15;
+            L.w.w1[i] = k < NFEAT ? p[OFF_W1 + h * NFEAT + k] : 0.0f;
+        }
+        for (int i = tid; i < NHID * NHID; i += TPB_T) L.w.w2[i] = p[OFF_W2 + i];
+    }
+    if (tid < NHID) {
+        L.b1[tid] = p[OFF_B1 + tid];
+        L.b2[tid] = p[OFF_B2 + tid];
+        L.w3[tid] = p[OFF_W3 + tid];
+    }
+}
+
 template <bool BF>
 __global__ __launch_bounds__(TPB_T) void k_mlp_grad(GradArgs a)
 {
-    __shared__ TrainLds L;
+    __shared__ TrainLds<BF> L;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, s = lane & 15;
-    for (int i = tid; i < NHID * 16; i += TPB_T) {
-        const int h = i >> 4, k = i & 15;
-        L.w1[i] = k < NFEAT ? a.p[OFF_W1 + h * NFEAT + k] : 0.0f;
-    }
-    for (int i = tid; i < NHID * NHID; i += TPB_T) L.w2[i] = a.p[OFF_W2 + i];
-    if (tid < NHID) {
-        L.b1[tid] = a.p[OFF_B1 + tid];
-        L.b2[tid] = a.p[OFF_B2 + tid];
-        L.w3[tid] = a.p[OFF_W3 + tid];
-    }
+    load_weights(L, a.p);
     const float b3 = a.p[OFF_B3];
     __syncthreads();
 
@@ -144,27 +233,30 @@ __global__ __launch_bounds__(TPB_T) void k_mlp_grad(GradArgs a)
 
     for (int tile = blockIdx.x * 4 + wave; tile < ntiles; tile += gridDim.x * 4) {
         const int64_t i = sample_index(a, (int64_t)tile * 16 + s);
-        f32x4 xb, xr;
+        // this lane's sample s, features 4 q ..; the last product wants the
+        // transpose (samples 4 q .., feature s), which goes through LDS rather
+        // than through a second gather (its sample indices cost a 64-bit
+        // remainder each)
+        f32x4 xb = {0.0f, 0.0f, 0.0f, 0.0f}, xr;
+        if (q < NFEAT / 4) xb = *(const f32x4*)&a.x[i * NFEAT + 4 * q];
+        *(f32x4*)&T1[s * 16 + 4 * q] = xb;
+        wave_lds_sync();
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int f = 4 * q + j;
-            xb[j] = f < NFEAT ? a.x[i * NFEAT + f] : 0.0f;
-            const int64_t ir = sample_index(a, (int64_t)tile * 16 + 4 * q + j);
-            xr[j] = s < NFEAT ? a.x[ir * NFEAT + s] : 0.0f;
-        }
+        for (int j = 0; j < 4; ++j) xr[j] = T1[(4 * q + j) * 16 + s];
+        wave_lds_sync();
+        const Frag<BF> xbf = frag<BF>(xb), xrf = frag<BF>(xr);
         // forward: H1^T = W1 X^T + b1, H2^T = W2 A1^T + b2
         f32x4 h1[4], a1[4], h2[4];
+        Frag<BF> a1f[4];
 #pragma unroll
         for (int hb = 0; hb < 4; ++hb) {
-            f32x4 w, c;
+            f32x4 c;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                w[j] = L.w1[(hb * 16 + s) * 16 + 4 * q + j];
-                c[j] = L.b1[hb * 16 + 4 * q + j];
-            }
-            h1[hb] = mma<BF>(L, wave, w, xb, c);
+            for (int j = 0; j < 4; ++j) c[j] = L.b1[hb * 16 + 4 * q + j];
+            h1[hb] = mma<BF>(L, wave, w1_frag(L, hb), xbf, c);
 #pragma unroll
             for (int j = 0; j < 4; ++j) a1[hb][j] = silu_hw(h1[hb][j]);
+            a1f[hb] = frag<BF>(a1[hb]);
         }
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
@@ -172,12 +264,7 @@ __global__ __launch_bounds__(TPB_T) void k_mlp_grad(GradArgs a)
 #pragma unroll
             for (int j = 0; j < 4; ++j) c[j] = L.b2[mb * 16 + 4 * q + j];
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb) {
-                f32x4 w;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) w[j] = L.w2[(mb * 16 + s) * NHID + kb * 16 + 4 * q + j];
-                c = mma<BF>(L, wave, w, a1[kb], c);
-            }
+            for (int kb = 0; kb < 4; ++kb) c = mma<BF>(L, wave, w2_frag(L, mb, kb), a1f[kb], c);
             h2[mb] = c;
         }
         float zp = 0.0f;
@@ -197,8 +284,9 @@ __global__ __launch_bounds__(TPB_T) void k_mlp_grad(GradArgs a)
 
         // backward through layer 3 and the second activation
         f32x4 dh2[4], dh1[4];
+        Frag<BF> dh2f[4];
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb)
+        for (int mb = 0; mb < 4; ++mb) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int h = mb * 16 + 4 * q + j;
@@ -206,17 +294,14 @@ __global__ __launch_bounds__(TPB_T) void k_mlp_grad(GradArgs a)
                 dh2[mb][j] = L.w3[h] * dz * dsilu_hw(h2[mb][j]);
                 gb2[mb][j] += dh2[mb][j];
             }
+            dh2f[mb] = frag<BF>(dh2[mb]);
+        }
         // dA1^T = W2^T dH2^T
 #pragma unroll
         for (int hb = 0; hb < 4; ++hb) {
             f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb) {
-                f32x4 w;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) w[j] = L.w2[(kb * 16 + 4 * q + j) * NHID + hb * 16 + s];
-                c = mma<BF>(L, wave, w, dh2[kb], c);
-            }
+            for (int kb = 0; kb < 4; ++kb) c = mma<BF>(L, wave, w2t_frag(L, hb, kb), dh2f[kb], c);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 dh1[hb][j] = c[j] * dsilu_hw(h1[hb][j]);
@@ -232,18 +317,14 @@ __global__ __launch_bounds__(TPB_T) void k_mlp_grad(GradArgs a)
                 T2[(b * 16 + 4 * q + j) * 16 + s] = dh2[b][j];
             }
         wave_lds_sync();
+        Frag<BF> a1t[4];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) a1t[nb] = frag<BF>(*(const f32x4*)&T1[(nb * 16 + s) * 16 + 4 * q]);
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
-            f32x4 A;
+            const Frag<BF> A = frag<BF>(*(const f32x4*)&T2[(mb * 16 + s) * 16 + 4 * q]);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) A[j] = T2[(mb * 16 + s) * 16 + 4 * q + j];
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                f32x4 B;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) B[j] = T1[(nb * 16 + s) * 16 + 4 * q + j];
-                gW2[mb][nb] = mma<BF>(L, wave, A, B, gW2[mb][nb]);
-            }
+            for (int nb = 0; nb < 4; ++nb) gW2[mb][nb] = mma<BF>(L, wave, A, a1t[nb], gW2[mb][nb]);
         }
         wave_lds_sync();
 #pragma unroll
@@ -253,10 +334,8 @@ __global__ __launch_bounds__(TPB_T) void k_mlp_grad(GradArgs a)
         wave_lds_sync();
 #pragma unroll
         for (int hb = 0; hb < 4; ++hb) {
-            f32x4 A;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) A[j] = T2[(hb * 16 + s) * 16 + 4 * q + j];
-            gW1[hb] = mma<BF>(L, wave, A, xr, gW1[hb]);
+            const Frag<BF> A = frag<BF>(*(const f32x4*)&T2[(hb * 16 + s) * 16 + 4 * q]);
+            gW1[hb] = mma<BF>(L, wave, A, xrf, gW1[hb]);
         }
         wave_lds_sync();
     }
@@ -328,25 +407,51 @@ struct ReduceArgs {
     int adam;
 };
 
+// FP64 sum of the workgroups' partial gradients in a fixed order, then Adam.
+// A workgroup takes RP parameters and splits the partials over RG groups of
+// threads, so that 317 workgroups are in flight and a thread's 16 loads are
+// all outstanding at once; with one thread per parameter, 20 workgroups each
+// waited for 256 loads in turn (74 us a step for 5 MB).
+constexpr int RP = 16, RG = TPB_T / RP;
+
 __global__ __launch_bounds__(TPB_T) void k_mlp_reduce(ReduceArgs a)
 {
-    const int i = blockIdx.x * TPB_T + threadIdx.x;
-    if (i == 0 && a.loss_out) {
-        double s = 0.0;
-        for (int k = 0; k < a.nparts; ++k) s += a.part_loss[k];
-        *a.loss_out = s;
+    __shared__ double red[RG][RP];
+    const int c = threadIdx.x & (RP - 1), g = threadIdx.x / RP;
+    const int i = blockIdx.x * RP + c;
+    const int per = (a.nparts + RG - 1) / RG, k0 = g * per, k1 = min(a.nparts, k0 + per);
+    double s = 0.0;
+    if (i < NPARAM) {
+#pragma unroll 16
+        for (int k = k0; k < k1; ++k) s += (double)a.part[(size_t)k * NPARAM + i];
     }
-    if (i >= NPARAM) return;
-    double g = 0.0;
-    for (int k = 0; k < a.nparts; ++k) g += (double)a.part[(size_t)k * NPARAM + i];
-    const float gf = (float)g;
-    if (a.grad) a.grad[i] = gf;
-    if (a.adam) {
-        const float m = a.beta1 * a.m[i] + (1.0f - a.beta1) * gf;
-        const float v = a.beta2 * a.v[i] + (1.0f - a.beta2) * gf * gf;
-        a.m[i] = m;
-        a.v[i] = v;
-        a.p[i] -= a.lr * (m / a.bc1) / (sqrtf(v / a.bc2) + a.eps);
+    red[g][c] = s;
+    __syncthreads();
+    if (g == 0 && i < NPARAM) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < RG; ++k) t += red[k][c];
+        const float gf = (float)t;
+        if (a.grad) a.grad[i] = gf;
+        if (a.adam) {
+            const float m = a.beta1 * a.m[i] + (1.0f - a.beta1) * gf;
+            const float v = a.beta2 * a.v[i] + (1.0f - a.beta2) * gf * gf;
+            a.m[i] = m;
+            a.v[i] = v;
+            a.p[i] -= a.lr * (m / a.bc1) / (sqrtf(v / a.bc2) + a.eps);
+        }
+    }
+    if (blockIdx.x == 0 && a.loss_out) {   // the loss: a sum over all threads' shares, in thread order
+        __shared__ double ls[TPB_T];
+        double v = 0.0;
+        for (int k = threadIdx.x; k < a.nparts; k += TPB_T) v += a.part_loss[k];
+        ls[threadIdx.x] = v;
+        __syncthreads();
+        for (int h = TPB_T / 2; h > 0; h >>= 1) {
+            if ((int)threadIdx.x < h) ls[threadIdx.x] += ls[threadIdx.x + h];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) *a.loss_out = ls[0];
     }
 }
 
@@ -543,7 +648,7 @@ lbm_status lbm_mlp_gradient(lbm_mlp* m, int64_t first, int32_t count, float c_le
         m->loss_cap = 1;
     }
     r.loss_out = m->loss;
-    k_mlp_reduce<<<(NPARAM + TPB_T - 1) / TPB_T, TPB_T, 0, m->stream>>>(r);
+    k_mlp_reduce<<<(NPARAM + RP - 1) / RP, TPB_T, 0, m->stream>>>(r);
     HCHK(hipGetLastError());
     if (grad) HCHK(hipMemcpyAsync(grad, m->grad, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, m->stream));
     double ls = 0.0;
@@ -588,7 +693,7 @@ lbm_status lbm_mlp_train(lbm_mlp* m, int32_t steps, int32_t batch, float lr, flo
         r.bc1 = (float)(1.0 - std::pow(0.9, (double)m->t));
         r.bc2 = (float)(1.0 - std::pow(0.999, (double)m->t));
         r.loss_out = m->loss + k;
-        k_mlp_reduce<<<(NPARAM + TPB_T - 1) / TPB_T, TPB_T, 0, m->stream>>>(r);
+        k_mlp_reduce<<<(NPARAM + RP - 1) / RP, TPB_T, 0, m->stream>>>(r);
     }
     HCHK(hipGetLastError());
     if (loss) {
