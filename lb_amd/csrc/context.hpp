@@ -19,6 +19,8 @@ struct lbm_ctx {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     size_t N = 0;              // padded cells
+    size_t NP = 0;             // population plane stride: N up to a whole cache line
+    bool rows_aligned = true;  // rows start on a cache line
     size_t NU = 0;             // caller's cells
     size_t elem = 0;           // bytes per stored population
     size_t rbytes = 0;         // bytes per arithmetic value
@@ -141,7 +143,7 @@ static inline void fill_common(const lbm_ctx* c, typename ST::T** p, typename ST
     K = make_consts<R>(c->d.compat);
     for (int k = 0; k < 4; ++k) rest[k] = ST::dev ? (R)(K.w[k] * (R)c->d.rho0) : R(0);
     typename ST::T* base = (typename ST::T*)c->pops;
-    for (int q = 0; q < Q; ++q) p[q] = base + (size_t)q * c->N;
+    for (int q = 0; q < Q; ++q) p[q] = base + (size_t)q * c->NP;
 }
 
 static inline MlpWeights closure_weights(const lbm_ctx* c)

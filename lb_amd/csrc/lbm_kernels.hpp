@@ -74,6 +74,10 @@ struct Geo {
     int ntx, nty;       // tiles along x and y
     int ntiles;
     int wx, wy, wz;     // index wrap per axis
+    int tx0, ty0, tz0;  // padded coordinates of the first tile: the box of non-solid cells
+    int tex, tey;       // its extents along x and y
+    int flat;           // no metadata: tile = 256 consecutive cells of the lattice
+    uint32_t rnx, rny;  // floor(2^32 / nx), floor(2^32 / ny)
 };
 
 // Boundary-node record on the device (padded coordinates).  Publish slots
@@ -245,8 +249,9 @@ __device__ __forceinline__ Cell cell_at(const Geo& g, int x, int y, int z)
     return c;
 }
 
-// Tiles cover the caller's cells only (halo cells are solid and never
-// collide).  Workgroups go to the XCDs in the hardware's round-robin order
+// Tiles cover the box of the non-solid cells only (solid cells never collide:
+// a cavity's 66-wide rows hold 64 fluid cells, one tile instead of three).
+// Workgroups go to the XCDs in the hardware's round-robin order
 // (workgroup b on XCD b mod 8), which keeps all of them on one narrow band of
 // each plane.  Where a row of tiles holds several tiles (ntx > 1), the tiles of
 // one row group are given workgroup ids that are equal mod 8: one XCD then
@@ -272,20 +277,46 @@ __device__ __forceinline__ int tile_of_block(const Geo& g, int b)
     return R * g.ntx + k;
 }
 
+// Where the whole lattice is one run of fluid cells (!FLAGS) whose rows do not
+// fill the tiles, a tile is 256 consecutive cells instead: no lane idles and
+// every access of the even step is whole cache lines, whatever the row length
+// (203 x 97 x 131, BF16: 131 -> 57 us a step; the 32-wide tiles of its rows
+// wrote partial lines with the streaming hint, 169 us on the even step).
+__device__ __forceinline__ uint32_t div_small(uint32_t n, uint32_t d, uint32_t rd, uint32_t& rem)
+{
+    uint32_t q = __umulhi(n, rd);   // n / d or one less
+    rem = n - q * d;
+    if (rem >= d) {
+        ++q;
+        rem -= d;
+    }
+    return q;
+}
+
+template <bool FLAGS>
 __device__ __forceinline__ Cell cell_of(const Geo& g)
 {
     Cell c;
-    const int t = tile_of_block(g, (int)blockIdx.x);
-    const int tx = t % g.ntx;
-    const int rem = t / g.ntx;
-    const int ty = rem % g.nty;
-    c.z = g.pz + rem / g.nty;
-    const int ux = (tx << g.bx_log2) + ((int)threadIdx.x & ((1 << g.bx_log2) - 1));
-    const int uy = ty * g.by + ((int)threadIdx.x >> g.bx_log2);
-    c.x = g.px + ux;
-    c.y = g.py + uy;
-    c.inside = ux < g.ux && uy < g.uy;
-    c.i = (uint32_t)(c.x + g.nx * (c.y + g.ny * c.z));
+    if (!FLAGS && g.flat) {
+        c.i = blockIdx.x * (uint32_t)TPB + threadIdx.x;
+        c.inside = c.i < (uint32_t)g.nx * (uint32_t)g.ny * (uint32_t)g.nz;
+        uint32_t x, y;
+        c.z = (int)div_small(div_small(c.i, (uint32_t)g.nx, g.rnx, x), (uint32_t)g.ny, g.rny, y);
+        c.x = (int)x;
+        c.y = (int)y;
+    } else {
+        const int t = tile_of_block(g, (int)blockIdx.x);
+        const int tx = t % g.ntx;
+        const int rem = t / g.ntx;
+        const int ty = rem % g.nty;
+        c.z = g.tz0 + rem / g.nty;
+        const int ex = (tx << g.bx_log2) + ((int)threadIdx.x & ((1 << g.bx_log2) - 1));
+        const int ey = ty * g.by + ((int)threadIdx.x >> g.bx_log2);
+        c.x = g.tx0 + ex;
+        c.y = g.ty0 + ey;
+        c.inside = ex < g.tex && ey < g.tey;
+        c.i = (uint32_t)(c.x + g.nx * (c.y + g.ny * c.z));
+    }
     set_deltas(g, c);
     return c;
 }
@@ -315,7 +346,8 @@ __device__ __forceinline__ void read_slot(const Cell& c, int q, bool odd, int& p
 
 // A wave's access to population q covers whole cache lines when it is not
 // shifted along x: every access of the even step, and on the odd step the
-// directions with c_x = 0 (tiles are whole rows or power-of-two segments).
+// directions with c_x = 0, if rows start on a line (the odd step's kernel is
+// compiled for both, NT = false where they do not).
 __host__ __device__ constexpr bool line_aligned(bool odd, int q) { return !odd || CX[q] == 0; }
 __host__ __device__ constexpr int read_plane(bool odd, int q) { return odd ? OPP[q] : q; }
 __device__ __forceinline__ uint32_t read_index(const Cell& c, bool odd, int q) { return odd ? nb(c, OPP[q]) : c.i; }
@@ -333,14 +365,14 @@ __device__ __forceinline__ typename ST::R reload_pop(typename ST::T* const* p, c
     return ST::template get<false>(p[read_plane(ODD, q)], read_index(c, ODD, q), rest[WCLASS[q]]);
 }
 
-template <class ST, bool ODD>
+template <class ST, bool ODD, bool NT = true>
 __device__ __forceinline__ void load_pop(typename ST::T* const* p, const typename ST::R* rest, const Cell& c,
                                          typename ST::R* f)
 {
 #pragma unroll
     for (int q = 0; q < Q; ++q)
         if (line_aligned(ODD, q))
-            f[q] = ST::template get<true>(p[read_plane(ODD, q)], read_index(c, ODD, q), rest[WCLASS[q]]);
+            f[q] = ST::template get<NT>(p[read_plane(ODD, q)], read_index(c, ODD, q), rest[WCLASS[q]]);
 #pragma unroll
     for (int q = 0; q < Q; ++q)
         if (!line_aligned(ODD, q))
@@ -522,7 +554,7 @@ __device__ __forceinline__ void stream_cell(const StepArgs<ST>& a, const Cell& c
 // INL: inlet rules deferred into this kernel (a separate instantiation: the
 // rule's code, even untaken, cost the obstacle workload's flagged step 1-2 %
 // in FP32/FP64 and 8 % in FP16 storage).
-template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC, bool INL>
+template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC, bool INL, bool NT>
 __device__ __forceinline__ void step_cells(const StepArgs<ST>& a)
 {
 #include "step_body.inc"
@@ -535,11 +567,11 @@ __device__ __forceinline__ void step_cells(const StepArgs<ST>& a)
 // before its stores (107 VGPRs) and ran 2.9 % faster on the periodic 256^3
 // workload (cumulant 2017: 3.2 %), while the 16-bit steps ran 2.1-2.6 %
 // slower that way and FP64 0.5 %.
-template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC = false, bool INL = false>
+template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC = false, bool INL = false, bool NT = true>
 __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
 {
     if constexpr (sizeof(typename ST::T) == 4) {
-        step_cells<ST, COLL, LIT, ODD, FLAGS, CC, INL>(a);
+        step_cells<ST, COLL, LIT, ODD, FLAGS, CC, INL, NT>(a);
     } else {
 #include "step_body.inc"
     }
@@ -553,7 +585,7 @@ __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
 template <class ST, int COLL, bool LIT, bool ODD, bool INL = false>
 __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(7, 7))) void k_step_w7(StepArgs<ST> a)
 {
-    step_cells<ST, COLL, LIT, ODD, true, false, INL>(a);
+    step_cells<ST, COLL, LIT, ODD, true, false, INL, true>(a);
 }
 
 // Moments, Smagorinsky rate and closure features of one cell, shared by the
@@ -611,7 +643,7 @@ __global__ __launch_bounds__(TPB) void k_step_mlp(MlpStepArgs<ST> ma)
     mlp_load_lds(L, ma.mlp);
     __syncthreads();
 
-    const Cell c = cell_of(a.g);
+    const Cell c = cell_of<FLAGS>(a.g);
     bool active = c.inside;
     uint8_t cls = CL_FLUID;
     if (FLAGS && active) cls = a.cls[c.i];

@@ -90,7 +90,8 @@ static lbm_status launch_steps(lbm_ctx* c, int nsteps)
                     if (odd) k_step<ST, COLL, false, true, true, true><<<grid, block, 0, c->stream>>>(a);
                     else k_step<ST, COLL, false, false, true, true><<<grid, block, 0, c->stream>>>(a);
                 } else {
-                    if (odd) k_step<ST, COLL, false, true, false, true><<<grid, block, 0, c->stream>>>(a);
+                    if (odd && !c->rows_aligned) k_step<ST, COLL, false, true, false, true, false, false><<<grid, block, 0, c->stream>>>(a);
+                    else if (odd) k_step<ST, COLL, false, true, false, true><<<grid, block, 0, c->stream>>>(a);
                     else k_step<ST, COLL, false, false, false, true><<<grid, block, 0, c->stream>>>(a);
                 }
             }
@@ -104,7 +105,8 @@ static lbm_status launch_steps(lbm_ctx* c, int nsteps)
                 if (odd) launch_flagged<ST, COLL, LIT, true, false>(grid, block, c->stream, a);
                 else launch_flagged<ST, COLL, LIT, false, false>(grid, block, c->stream, a);
             } else {
-                if (odd) k_step<ST, COLL, LIT, true, false><<<grid, block, 0, c->stream>>>(a);
+                if (odd && !c->rows_aligned) k_step<ST, COLL, LIT, true, false, false, false, false><<<grid, block, 0, c->stream>>>(a);
+                else if (odd) k_step<ST, COLL, LIT, true, false><<<grid, block, 0, c->stream>>>(a);
                 else k_step<ST, COLL, LIT, false, false><<<grid, block, 0, c->stream>>>(a);
             }
         }
