@@ -13,6 +13,12 @@
 
 using namespace lbm;
 
+// pinned ring of the read-backs (readback.hpp): most slots, bytes of a slot,
+// bytes that another thread is worth
+static constexpr int RB_SLOTS = 16;
+static constexpr size_t RB_SLOT = 1 << 20;
+static constexpr size_t RB_PER_THREAD = 2 << 20;
+
 struct lbm_ctx {
     lbm_desc d;
     int device = 0;
@@ -78,6 +84,10 @@ struct lbm_ctx {
     void* uerr = nullptr;           // previous velocity, 3 planes of the arithmetic type, caller layout
     // per-block partials of a diagnostics step go here instead of `partials` when set
     double* diag_dst = nullptr;
+    // read-backs
+    char* rb_host = nullptr;          // pinned, rb_slots slots of RB_SLOT bytes
+    int rb_slots = 0;
+    hipEvent_t rb_ev[RB_SLOTS] = {};
     // asynchronous snapshots: rho, u, omega into snap_dev on the context stream,
     // then a copy to pinned host memory on copy_stream while steps go on
     double* snap_dev = nullptr;       // 5 planes FP64, caller layout

@@ -19,6 +19,7 @@
 
 #include "../../include/lbm_closure.h"
 #include "context.hpp"
+#include "readback.hpp"
 
 using namespace lbm;
 
@@ -525,6 +526,9 @@ void lbm_destroy(lbm_ctx* c)
         if (b) (void)hipFree(b);
     if (c->snap_pending && c->ev_snap_copy) (void)hipEventSynchronize(c->ev_snap_copy);
     if (c->snap_host) (void)hipHostFree(c->snap_host);
+    if (c->rb_host) (void)hipHostFree(c->rb_host);
+    for (hipEvent_t e : c->rb_ev)
+        if (e) (void)hipEventDestroy(e);
     if (c->ev_snap) (void)hipEventDestroy(c->ev_snap);
     if (c->ev_snap_copy) (void)hipEventDestroy(c->ev_snap_copy);
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
@@ -882,13 +886,14 @@ lbm_status lbm_moment_avg(lbm_ctx* c, double* rho, double* ux, double* uy, doubl
     lbm_status st = avg_flush(c);
     if (st != LBM_OK) return st;
     double* outs[4] = {rho, ux, uy, uz};
+    // momentAvg (MomentTimeAvg.h:47-77): the sums divided by the counter
+    const double n = (double)c->avg_count;
+    if (ring_ready(c)) return read_planes(c, c->avg, outs, 4, n);
     for (int k = 0; k < 4; ++k)
         if (outs[k])
             HIPCHK(hipMemcpyAsync(outs[k], c->avg + k * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost,
                                   c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    // momentAvg (MomentTimeAvg.h:47-77): the sums divided by the counter
-    const double n = (double)c->avg_count;
     for (int k = 0; k < 4; ++k)
         if (outs[k])
             for (size_t i = 0; i < c->NU; ++i) outs[k][i] /= n;
@@ -962,9 +967,17 @@ lbm_status lbm_get_macroscopic(lbm_ctx* c, double* rho, double* ux, double* uy, 
     if (!c->initialized) return LBM_E_STATE;
     lbm_status st = lbm_sync(c);
     if (st != LBM_OK && st != LBM_E_NAN) return st;
+    double* outs[4] = {rho, ux, uy, uz};
+    if (ring_ready(c))
+        return with_storage(c, [&](auto stv) -> lbm_status {
+            using ST = decltype(stv);
+            using R = typename ST::R;
+            k_macro<ST, R><<<blocks_for(c->NU), TPB, 0, c->stream>>>(aux_args<ST>(c));
+            HIPCHK(hipGetLastError());
+            return read_planes(c, (const R*)c->stage, outs, 4);
+        });
     st = run_macro(c);
     if (st != LBM_OK) return st;
-    double* outs[4] = {rho, ux, uy, uz};
     for (int k = 0; k < 4; ++k)
         if (outs[k])
             HIPCHK(hipMemcpyAsync(outs[k], c->stage + k * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost,
@@ -1060,6 +1073,7 @@ lbm_status lbm_get_omega(lbm_ctx* c, double* omega)
         st = run_macro(c);
     }
     if (st != LBM_OK) return st;
+    if (ring_ready(c)) return read_planes(c, c->stage + 4 * c->NU, &omega, 1);
     HIPCHK(hipMemcpyAsync(omega, c->stage + 4 * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1133,6 +1147,7 @@ lbm_status lbm_get_population(lbm_ctx* c, int32_t q, double* f)
         return LBM_OK;
     });
     if (st != LBM_OK) return st;
+    if (ring_ready(c)) return read_planes(c, c->stage, &f, 1);
     HIPCHK(hipMemcpyAsync(f, c->stage, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1154,8 +1169,13 @@ lbm_status lbm_get_populations(lbm_ctx* c, double* f)
             return LBM_OK;
         });
         if (st != LBM_OK) return st;
-        HIPCHK(hipMemcpyAsync(f + (size_t)q * c->NU, c->stage, c->NU * sizeof(double), hipMemcpyDeviceToHost,
-                              c->stream));
+        double* fq = f + (size_t)q * c->NU;
+        if (ring_ready(c)) {
+            st = read_planes(c, c->stage, &fq, 1);
+            if (st != LBM_OK) return st;
+            continue;
+        }
+        HIPCHK(hipMemcpyAsync(fq, c->stage, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;

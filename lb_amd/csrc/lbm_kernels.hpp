@@ -1139,26 +1139,27 @@ __device__ __forceinline__ void cell_macro(const AuxArgs<ST>& a, const Cell& c, 
 }
 
 // rho, u and omega of the current state into 5 FP64 staging planes.
-template <class ST>
+template <class ST, class O = double>
 __global__ __launch_bounds__(TPB) void k_macro(AuxArgs<ST> a)
 {
     using R = typename ST::R;
+    O* io = (O*)a.io;
     uint32_t iu;
     Cell c;
     if (!user_cell(a.g, iu, c)) return;
     const size_t NU = (size_t)a.g.ux * a.g.uy * a.g.uz;
     const uint8_t cls = a.cls[c.i];
     if (cls == CL_SOLID) {
-        for (int k = 0; k < 5; ++k) a.io[k * NU + iu] = 0.0;
+        for (int k = 0; k < 5; ++k) io[k * NU + iu] = O(0);
         return;
     }
     R rho, ux, uy, uz, om;
     cell_macro(a, c, cls, rho, ux, uy, uz, &om);
-    a.io[iu] = (double)rho;
-    a.io[NU + iu] = (double)ux;
-    a.io[2 * NU + iu] = (double)uy;
-    a.io[3 * NU + iu] = (double)uz;
-    a.io[4 * NU + iu] = (double)om;
+    io[iu] = (O)rho;
+    io[NU + iu] = (O)ux;
+    io[2 * NU + iu] = (O)uy;
+    io[3 * NU + iu] = (O)uz;
+    io[4 * NU + iu] = (O)om;
 }
 
 // MomentTimeAvg::momentAdd as its own pass: rho, u of the current state (the
