@@ -84,7 +84,8 @@ namespace {
 struct Layout {
     int ux, uy, uz;   // caller's lattice
     int px, py, pz;   // halo per axis
-    int nx, ny, nz;   // padded
+    int nx, ny, nz;   // padded: row pitch, rows, planes
+    size_t n;         // cells of a plane array
     bool w[3];
     size_t user(int x, int y, int z) const
     {
@@ -148,7 +149,7 @@ NodeDev node_dev(const Layout& L, const lbm_bc_node& b)
 static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
 {
     const size_t NU = (size_t)L.ux * L.uy * L.uz;
-    const size_t N = (size_t)L.nx * L.ny * L.nz;
+    const size_t N = L.n;
     std::vector<uint8_t> kind(NU);
     for (size_t i = 0; i < NU; ++i) {
         const int F = d->flags[i];
@@ -571,11 +572,13 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     L.w[2] = d->periodic[2] != 0;
     const size_t elem = d->storage == LBM_STORAGE_F64 ? 8 : d->storage == LBM_STORAGE_F32 ? 4 : 2;
     const int line = (int)(128 / elem);   // populations per 128-byte cache line
-    // A halo along x is a whole line of solid cells on each side, so that the
-    // caller's rows start on a line and the step's line-aligned accesses are
-    // aligned in fact; only its innermost cells are ever read.
-    // The line starts at the first cell of the box of non-solid cells, which is
-    // where the step's tiles start.
+    // Along an axis without index wrap the non-solid cells have a halo cell on
+    // each side.  The box of non-solid cells, which is what the step's tiles
+    // cover, starts a cache line; its left halo is the last cell of the line
+    // before, which the row before ends in: a row takes no line of its own for
+    // it (and may not be longer than the pitch, nor may its two halo cells meet).
+    // With a line of its own on each side: 210 x 101 x 92 duct, FP16, 5 lines a row
+    // instead of 4; 128-wide cavity, FP32, 6 instead of 5.
     int lo[3] = {L.ux, L.uy, L.uz}, hi[3] = {-1, -1, -1};
     {
         const int32_t* f = d->flags;
@@ -601,10 +604,13 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     L.px = L.w[0] ? 0 : line - lo[0] % line;
     L.py = L.w[1] ? 0 : 1;
     L.pz = L.w[2] ? 0 : 1;
-    L.nx = L.w[0] ? L.ux : (L.px + L.ux + 1 + line - 1) / line * line;
+    L.nx = L.w[0] ? L.ux : (std::max(L.ux, hi[0] - lo[0] + 3) + line - 1) / line * line;
     L.ny = L.uy + 2 * L.py;
     L.nz = L.uz + 2 * L.pz;
-    const size_t N = (size_t)L.nx * L.ny * L.nz;
+    // the last row's cells and right halo may lie past its pitch
+    const size_t N = (size_t)L.nx * L.ny * L.nz +
+                     (L.w[0] ? 0 : (size_t)std::max(0, L.px + std::max(L.ux, hi[0] + 2) - L.nx));
+    L.n = N;
     const size_t NP = (N + line - 1) / line * line;
     const size_t NU = (size_t)L.ux * L.uy * L.uz;
     if (N * elem > 0xFFFFFFFFull || N >= 0x7FFFFFFFull) return LBM_E_ARG;  // 32-bit plane offsets
@@ -680,6 +686,7 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     c->g.nx = L.nx;
     c->g.ny = L.ny;
     c->g.nz = L.nz;
+    c->g.n = (uint32_t)N;
     c->g.px = L.px;
     c->g.py = L.py;
     c->g.pz = L.pz;

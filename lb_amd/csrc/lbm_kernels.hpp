@@ -10,8 +10,8 @@
 // which reads and writes two full lattices plus rho/u/omega every step.
 //
 // A-A layout: one population array P[q][cell] (structure of arrays, x
-// fastest, a solid halo on every non-periodic axis: one cell in y and z, a
-// whole cache line of cells in x so that rows start on a line).  With t the
+// fastest, a solid halo on every non-periodic axis: one cell in y and z, in x
+// one on each side inside whole cache lines, so that rows start on a line).  With t the
 // number of completed steps:
 //   even t: cell x reads f_q from P[q][x] and writes post-collision f*_q to
 //           P[opp q][x];
@@ -66,9 +66,10 @@ constexpr int NW_CUM2017 = 62;
 constexpr int PUB_MAC = 4;   // published rho, ux, uy, uz per publish slot
 
 struct Geo {
-    int nx, ny, nz;     // padded lattice
-    int px, py, pz;     // offset of the caller's lattice: halo width per axis (0 on
-                        // index-wrap axes; along x a whole cache line of solid cells)
+    int nx, ny, nz;     // padded lattice: row pitch, rows, planes
+    int px, py, pz;     // offset of the caller's lattice (0 on index-wrap axes); px + x may
+                        // pass the row pitch: a row's left halo lies in the line before it
+    uint32_t n;         // cells of a plane array
     int ux, uy, uz;     // caller's lattice
     int bx_log2, by;    // tile: (1 << bx_log2) x by cells, 256 threads
     int ntx, nty;       // tiles along x and y
@@ -664,7 +665,7 @@ __global__ __launch_bounds__(TPB) void k_step_mlp(MlpStepArgs<ST> ma)
         } else {
             load_pop<ST, ODD>(a.p, a.rest, c, f);
         }
-        closure_prep<ST>(f, a.first != 0, a.macro, (size_t)a.g.nx * a.g.ny * a.g.nz, c.i, a.tau, a.cles, L, cp);
+        closure_prep<ST>(f, a.first != 0, a.macro, (size_t)a.g.n, c.i, a.tau, a.cles, L, cp);
         if (cp.env) {
 #pragma unroll
             for (int k = 0; k < NFEAT; ++k) xn[k] = cp.xn[k];
@@ -908,9 +909,10 @@ __global__ __launch_bounds__(TPB) void k_periodic(PatchArgs<ST> a)
     const uint32_t pi = (uint32_t)b.partner;
     const bool self_partner = pi == c.i;
     const uint8_t pcls = a.cls[pi];
-    const int px = (int)(pi % (uint32_t)a.g.nx);
-    const int py = (int)((pi / (uint32_t)a.g.nx) % (uint32_t)a.g.ny);
-    const int pz = (int)(pi / ((uint32_t)a.g.nx * (uint32_t)a.g.ny));
+    const uint32_t pr = pi - (uint32_t)a.g.px;   // rows from their first caller's cell
+    const int px = (int)(pr % (uint32_t)a.g.nx) + a.g.px;
+    const int py = (int)((pr / (uint32_t)a.g.nx) % (uint32_t)a.g.ny);
+    const int pz = (int)(pr / ((uint32_t)a.g.nx * (uint32_t)a.g.ny));
     const Cell pc = cell_at(a.g, px, py, pz);
     const R* post = a.pub_post + (size_t)b.s0 * Q;
 #pragma unroll
@@ -1019,7 +1021,7 @@ template <class ST>
 __global__ __launch_bounds__(TPB) void k_init(AuxArgs<ST> a)
 {
     using R = typename ST::R;
-    const size_t N = (size_t)a.g.nx * a.g.ny * a.g.nz;
+    const size_t N = (size_t)a.g.n;
     const size_t ii = (size_t)blockIdx.x * TPB + threadIdx.x;
     if (ii >= N) return;
     const uint32_t i = (uint32_t)ii;
@@ -1094,7 +1096,7 @@ __device__ __forceinline__ void cell_macro(const AuxArgs<ST>& a, const Cell& c, 
     using R = typename ST::R;
     R f[Q];
     cell_state(a, c, cls, f);
-    const size_t N = (size_t)a.g.nx * a.g.ny * a.g.nz;
+    const size_t N = (size_t)a.g.n;
     if (a.lit) {
         if (a.first) {
             rho = a.macro[c.i];
@@ -1324,7 +1326,7 @@ __global__ __launch_bounds__(TPB) void k_closure_eval(ClosureEvalArgs<ST> e)
     if (active) {
         R f[Q];
         cell_state(a, c, a.cls[c.i], f);
-        closure_prep<ST>(f, a.first != 0, a.macro, (size_t)a.g.nx * a.g.ny * a.g.nz, c.i, a.tau, a.cles, L, cp);
+        closure_prep<ST>(f, a.first != 0, a.macro, (size_t)a.g.n, c.i, a.tau, a.cles, L, cp);
         if (cp.env) {
 #pragma unroll
             for (int k = 0; k < NFEAT; ++k) xn[k] = cp.xn[k];
@@ -1367,7 +1369,7 @@ __global__ __launch_bounds__(TPB) void k_filter(AuxArgs<ST> a, int fct, int cx, 
                 if (cls == CL_SOLID) continue;
                 R rho, ux, uy, uz;
                 if (a.first) {
-                    const size_t N = (size_t)a.g.nx * a.g.ny * a.g.nz;
+                    const size_t N = (size_t)a.g.n;
                     rho = a.macro[c.i];
                     ux = a.macro[N + c.i];
                     uy = a.macro[2 * N + c.i];
