@@ -567,7 +567,10 @@ __device__ __forceinline__ void step_cells(const StepArgs<ST>& a)
 // even FP32 step through step_cells computes all 27 post-collision values
 // before its stores (107 VGPRs) and ran 2.9 % faster on the periodic 256^3
 // workload (cumulant 2017: 3.2 %), while the 16-bit steps ran 2.1-2.6 %
-// slower that way and FP64 0.5 %.
+// slower that way and FP64 0.5 %.  No launch bound holds the 16-bit steps to more
+// waves: they need 64 VGPRs with the cumulant operators (8 waves), and a hint for
+// 7 made BGK and the 2017 operators spill 650 bytes a lane (210 x 101 x 92 duct,
+// FP16, 2017: 140 -> 95 us a step without it).
 template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC = false, bool INL = false, bool NT = true>
 __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
 {
@@ -576,17 +579,6 @@ __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
     } else {
 #include "step_body.inc"
     }
-}
-
-// The boundary-aware step for 16-bit storage, held to 7 waves per SIMD (72
-// VGPRs instead of 75-76, which allow 6).  A 16-bit wave moves half the bytes
-// of an FP32 one, so it needs more waves in flight: on the obstacle workload
-// the step took 2 % less time.  FP32 was unchanged, and 8 waves spilled and
-// ran 7 % slower.
-template <class ST, int COLL, bool LIT, bool ODD, bool INL = false>
-__global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(7, 7))) void k_step_w7(StepArgs<ST> a)
-{
-    step_cells<ST, COLL, LIT, ODD, true, false, INL, true>(a);
 }
 
 // Moments, Smagorinsky rate and closure features of one cell, shared by the
