@@ -33,6 +33,7 @@ struct lbm_ctx {
     Geo g{};
     bool flags_needed = false; // any non-fluid cell (halo included)
     int n_inlet = 0, n_eq = 0, n_outlet = 0, n_ghost = 0, n_pub = 0;
+    int n_interp = 0;             // interpolated outlet entries
     int n_upd = 0;                // moving-wall and Zou-He inlet entries
     std::vector<int> ghost_off;  // launch boundaries of the ghost list (dependency levels)
     void* pops = nullptr;
@@ -245,15 +246,18 @@ static inline lbm_status launch_patches(lbm_ctx* c, int odd_next)
         u.pub_post = (const typename ST::R*)c->inl_post;
         k_inlet_state<ST><<<blocks_for(u.n), TPB, 0, c->stream>>>(u);
     }
-    if (c->n_eq) {
+    const int n_interp = c->outl_deferred ? 0 : c->n_interp;
+    if (c->n_eq || n_interp) {
         a.nodes = c->inl;
-        a.n = c->n_inlet;
-        k_inlet_eq<ST><<<blocks_for(a.n), TPB, 0, c->stream>>>(a);
+        a.n = c->n_eq ? c->n_inlet : 0;
+        const int bi = (a.n + NODES_PER_BLOCK - 1) / NODES_PER_BLOCK;
+        const int no = n_interp ? c->n_outlet : 0;
+        k_inlet_outlet<ST><<<bi + (no + NODES_PER_BLOCK - 1) / NODES_PER_BLOCK, TPB, 0, c->stream>>>(a, c->outl, no, bi);
     }
-    if (c->n_outlet && !c->outl_deferred) {
+    if (c->n_outlet > c->n_interp) {
         a.nodes = c->outl;
         a.n = c->n_outlet;
-        k_outlet<ST><<<blocks_for(a.n), TPB, 0, c->stream>>>(a);
+        k_outlet_eq<ST><<<blocks_for(a.n), TPB, 0, c->stream>>>(a);
     }
     for (size_t l = 0; l + 1 < c->ghost_off.size(); ++l) {
         a.nodes = c->ghost + c->ghost_off[l];

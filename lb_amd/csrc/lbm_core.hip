@@ -167,17 +167,20 @@ static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
     P.ghost.clear();
     P.n_eq = 0;
     P.n_pub = 0;
-    auto pub_slot = [&](size_t iu) -> int32_t {
+    // publish slot of a cell; post: its post-collision populations are read too
+    std::vector<uint8_t> pub_post(NU, 0);
+    auto pub_slot = [&](size_t iu, bool post) -> int32_t {
         if (pub_of[iu] < 0) pub_of[iu] = P.n_pub++;
+        if (post) pub_post[iu] = 1;
         return pub_of[iu];
     };
     // slot of a neighbour whose rho/u/f* a patch reads: -1 for solid cells
     // (zero in the reference), error for inlet cells (not published here)
-    auto ref_slot = [&](int x, int y, int z, int32_t& slot) -> lbm_status {
+    auto ref_slot = [&](int x, int y, int z, int32_t& slot, bool post) -> lbm_status {
         const size_t j = L.user(x, y, z);
         if (kind[j] == K_SOLID) slot = -1;
         else if (kind[j] == K_INLET) return LBM_E_UNSUPPORTED;
-        else slot = pub_slot(j);
+        else slot = pub_slot(j, post);
         return LBM_OK;
     };
 
@@ -207,8 +210,8 @@ static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
                 int x1, y1, z1, x2, y2, z2;
                 if (sx != 0 && L.nbr(b.x, b.y, b.z, -sx, 0, 0, x1, y1, z1) &&
                     L.nbr(b.x, b.y, b.z, -2 * sx, 0, 0, x2, y2, z2)) {
-                    lbm_status st = ref_slot(x1, y1, z1, e.s0);
-                    if (st == LBM_OK) st = ref_slot(x2, y2, z2, e.s1);
+                    lbm_status st = ref_slot(x1, y1, z1, e.s0, false);
+                    if (st == LBM_OK) st = ref_slot(x2, y2, z2, e.s1, false);
                     if (st != LBM_OK) return st;
                     P.n_eq++;
                 } else {
@@ -227,10 +230,10 @@ static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
                          : (b.nx == -1.0f && b.ny == 0.0f && b.nz == 0.0f) ? -1 : 0;
             if (sx == 0) break;   // other normals: no action (OutletDensityInterpolated.h:249)
             NodeDev e = node_dev(L, b);
-            e.s0 = pub_slot(i);
+            e.s0 = pub_slot(i, true);
             int xu, yu, zu;
             if (L.nbr(b.x, b.y, b.z, -sx, 0, 0, xu, yu, zu)) {
-                lbm_status st = ref_slot(xu, yu, zu, e.s1);
+                lbm_status st = ref_slot(xu, yu, zu, e.s1, true);
                 if (st != LBM_OK) return st;
             } else {
                 e.s1 = -2;   // only the irregular-node copy applies
@@ -256,7 +259,7 @@ static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
             if (kind[i] == K_INLET || has_outlet[i]) return LBM_E_UNSUPPORTED;
             has_outlet[i] = 1;
             NodeDev e = node_dev(L, b);
-            e.s0 = pub_slot(i);   // the node's own rho, u
+            e.s0 = pub_slot(i, false);   // the node's own rho, u
             uint32_t mask = 0;
             if (b.kind != LBM_BC_OUTLET_EQUILIBRIUM) {
                 for (int q = 0; q < Q; ++q) {
@@ -268,7 +271,7 @@ static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
                     const size_t j = L.user(x1, y1, z1);
                     if (!b.regular && !(d->flags[j] > 0)) continue;
                     if (kind[j] == K_INLET) return LBM_E_UNSUPPORTED;
-                    if (kind[j] != K_SOLID) pub_slot(j);
+                    if (kind[j] != K_SOLID) pub_slot(j, false);
                     mask |= 1u << q;
                 }
             }
@@ -290,7 +293,7 @@ static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
             const int qx = axis == 0 ? b.per_idx : b.x, qy = axis == 1 ? b.per_idx : b.y,
                       qz = axis == 2 ? b.per_idx : b.z;
             e.partner = (int32_t)L.pad(qx, qy, qz);
-            e.s0 = b.regular ? -1 : pub_slot(i);
+            e.s0 = b.regular ? -1 : pub_slot(i, true);
             P.ghost.push_back(e);
             break;
         }
@@ -427,6 +430,7 @@ static lbm_status classify(const lbm_desc* d, const Layout& L, Plan& P)
                 // is not 1 (CollisionCumD3Q27TurbulentCombined.h:1071-1076)
                 const bool c17 = d->collision == LBM_COLLISION_COMBINED && d->flags[iu] != 1;
                 P.node[ip] = (uint64_t)S | ((uint64_t)K << 32) | ((uint64_t)c17 << NW_CUM2017) |
+                             ((uint64_t)(pub_of[iu] >= 0 && !pub_post[iu]) << NW_MAC_ONLY) |
                              ((uint64_t)wall[iu] << 63);
                 if (kind[iu] == K_INLET) {
                     P.cls[ip] = CL_INLET;
@@ -641,6 +645,8 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     for (const NodeDev& e : P.inl)
         if (e.kind == LBM_BC_INLET_MOVING_WALL || e.kind == LBM_BC_INLET_ZOU_HE) c->n_upd++;
     c->n_outlet = (int)P.outl.size();
+    for (const NodeDev& e : P.outl)
+        if (e.kind == LBM_BC_OUTLET_INTERPOLATED) c->n_interp++;
     if (d->outlet_sponge) {
         // OutletNeighbourEquilibriumOmega::outletOmega (:18-79): the first outlet
         // entry's normal picks the axis; the last ceil(0.1 n) cells of it

@@ -63,6 +63,9 @@ constexpr int TPB = 256;
 // bit 62 the Combined operator's 2017 branch (flag != 1), bit 63 wall-list node
 constexpr uint64_t MASK27 = (1ull << 27) - 1;
 constexpr int NW_CUM2017 = 62;
+// bit 61: of a publishing cell only rho and u are read (equilibrium inlets and
+// outlets), not its post-collision populations
+constexpr int NW_MAC_ONLY = 61;
 constexpr int PUB_MAC = 4;   // published rho, ux, uy, uz per publish slot
 
 struct Geo {
@@ -143,6 +146,21 @@ __device__ __forceinline__ R sponge(R omega, int axis, int begin, R deriv, const
     return omega - deriv * (R)(v - begin);
 }
 
+// rho and u as the rule forms them, u with the outlet's density.
+template <class R>
+__device__ __forceinline__ void outlet_moments(const R* d, R density, R& rho, R& ux, R& uy, R& uz)
+{
+    LBM_FP_STRICT
+    rho = d[0] + d[1] + d[2] + d[3] + d[4] + d[5] + d[6] + d[7] + d[8] + d[9] + d[10] + d[11] + d[12] + d[13] +
+          d[14] + d[15] + d[16] + d[17] + d[18] + d[19] + d[20] + d[21] + d[22] + d[23] + d[24] + d[25] + d[26];
+    ux = (d[1] - d[2] + d[7] - d[8] + d[9] - d[10] - d[11] + d[12] - d[15] + d[16] - d[19] + d[20] - d[21] + d[22] +
+          d[23] - d[24] - d[25] + d[26]) / density;
+    uy = (-d[5] + d[6] - d[11] + d[12] + d[13] - d[14] + d[15] - d[16] + d[17] - d[18] + d[19] - d[20] - d[21] +
+          d[22] - d[23] + d[24] - d[25] + d[26]) / density;
+    uz = (-d[3] + d[4] - d[7] + d[8] + d[9] - d[10] - d[13] + d[14] + d[17] - d[18] - d[19] + d[20] + d[21] - d[22] -
+          d[23] + d[24] - d[25] + d[26]) / density;
+}
+
 // OutletDensityInterpolated::outlet (OutletDensityInterpolated.h:170-252) on
 // one node: interpolated incoming populations, then the density reset.
 // The interpolated rule itself on the node's current populations d (the
@@ -169,15 +187,7 @@ __device__ __forceinline__ bool outlet_blend(R* d, const NodeDev& b, const R* pu
             d[vel] = cs * up + (R(1) - cs) * self[vel];
         }
     }
-    const R density = b.rho;
-    rho = d[0] + d[1] + d[2] + d[3] + d[4] + d[5] + d[6] + d[7] + d[8] + d[9] + d[10] + d[11] + d[12] + d[13] +
-          d[14] + d[15] + d[16] + d[17] + d[18] + d[19] + d[20] + d[21] + d[22] + d[23] + d[24] + d[25] + d[26];
-    ux = (d[1] - d[2] + d[7] - d[8] + d[9] - d[10] - d[11] + d[12] - d[15] + d[16] - d[19] + d[20] - d[21] + d[22] +
-          d[23] - d[24] - d[25] + d[26]) / density;
-    uy = (-d[5] + d[6] - d[11] + d[12] + d[13] - d[14] + d[15] - d[16] + d[17] - d[18] + d[19] - d[20] - d[21] +
-          d[22] - d[23] + d[24] - d[25] + d[26]) / density;
-    uz = (-d[3] + d[4] - d[7] + d[8] + d[9] - d[10] - d[13] + d[14] + d[17] - d[18] - d[19] + d[20] + d[21] - d[22] -
-          d[23] + d[24] - d[25] + d[26]) / density;
+    outlet_moments<R>(d, b.rho, rho, ux, uy, uz);
     return true;
 }
 
@@ -535,9 +545,11 @@ __device__ __forceinline__ void stream_cell(const StepArgs<ST>& a, const Cell& c
             a.pub_mac[(size_t)bi * PUB_MAC + 1] = ux;
             a.pub_mac[(size_t)bi * PUB_MAC + 2] = uy;
             a.pub_mac[(size_t)bi * PUB_MAC + 3] = uz;
-            R* dst = a.pub_post + (size_t)bi * Q;
+            if (!((nw >> NW_MAC_ONLY) & 1u)) {
+                R* dst = a.pub_post + (size_t)bi * Q;
 #pragma unroll
-            for (int q = 0; q < Q; ++q) dst[q] = P[q];
+                for (int q = 0; q < Q; ++q) dst[q] = P[q];
+            }
         }
     }
     // streaming writes, shared by every lane of the wave (boundary lanes drop
@@ -746,14 +758,12 @@ __device__ __forceinline__ void store_node(const PatchArgs<ST>& a, const typenam
 // steady x-momentum balance d(rho/3)/dx = nu d2u/dx2); the reference's
 // nu/3, and its sign on the +x branch (:80), under LBM_COMPAT_INLETRHO.
 template <class ST>
-__global__ __launch_bounds__(TPB) void k_inlet_eq(PatchArgs<ST> a)
+__device__ __forceinline__ void inlet_eq(const PatchArgs<ST>& a, int j, int q)
 {
     LBM_FP_STRICT
     using R = typename ST::R;
-    const int j = blockIdx.x * TPB + threadIdx.x;
-    if (j >= a.n) return;
     const NodeDev b = a.nodes[j];
-    if (b.kind != LBM_BC_INLET_EQUILIBRIUM) return;
+    if (b.kind != LBM_BC_INLET_EQUILIBRIUM || q >= Q) return;
     const R uxb = b.ux, uyb = b.uy, uzb = b.uz;
     const R rho1 = b.s0 >= 0 ? a.pub_mac[(size_t)b.s0 * PUB_MAC] : R(0);
     const R ux1 = b.s0 >= 0 ? a.pub_mac[(size_t)b.s0 * PUB_MAC + 1] : R(0);
@@ -770,8 +780,7 @@ __global__ __launch_bounds__(TPB) void k_inlet_eq(PatchArgs<ST> a)
     } else {
         return;
     }
-#pragma unroll
-    for (int q = 0; q < Q; ++q) a.inl_state[(size_t)j * Q + q] = feq_q(a.K, q, uxb, uyb, uzb, rhob);
+    a.inl_state[(size_t)j * Q + q] = feq_q(a.K, q, uxb, uyb, uzb, rhob);
 }
 
 // State update of moving-wall and Zou-He inlet cells (the rules of
@@ -861,24 +870,84 @@ __device__ __forceinline__ void outlet_equilibrium(const PatchArgs<ST>& a, const
 }
 
 template <class ST>
-__global__ __launch_bounds__(TPB) void k_outlet(PatchArgs<ST> a)
+__global__ __launch_bounds__(TPB) void k_outlet_eq(PatchArgs<ST> a)
 {
-    LBM_FP_STRICT
-    using R = typename ST::R;
     const int j = blockIdx.x * TPB + threadIdx.x;
     if (j >= a.n) return;
     const NodeDev b = a.nodes[j];
-    if (b.kind != LBM_BC_OUTLET_INTERPOLATED) {
-        outlet_equilibrium(a, b);
+    if (b.kind != LBM_BC_OUTLET_INTERPOLATED) outlet_equilibrium(a, b);
+}
+
+// Equilibrium inlets (entries [0, a.n) of a.nodes, the first inlet_blocks
+// workgroups) and interpolated outlets (outl, the other workgroups) in one
+// launch: they read the step's records and write their own cells only.
+//
+// What bounds it is the number of cache lines: a node of an x-plane has each of
+// its populations on a line of its own.  32 lanes share a node, one population
+// each, so that a wave asks for 54 lines at once and the records and the inlet
+// state (27 values in a row) are one or two lines; with one thread a node a wave
+// asked for 64 lines 27 times over, on 37 of the CUs.  9292 nodes of each kind,
+// FP16: 26.5 + 4.8 us in two launches -> 17.0 in one.
+// Sums keep the rule's order: every lane forms them from LDS.
+constexpr int NODE_LANES = 32;
+constexpr int NODES_PER_BLOCK = TPB / NODE_LANES;
+
+template <class ST>
+__global__ __launch_bounds__(TPB) void k_inlet_outlet(PatchArgs<ST> a, const NodeDev* outl, int n_outl,
+                                                      int inlet_blocks)
+{
+    LBM_FP_STRICT
+    using R = typename ST::R;
+    __shared__ R sh[NODES_PER_BLOCK][NODE_LANES];
+    const int g = (int)threadIdx.x / NODE_LANES, q = (int)threadIdx.x % NODE_LANES;
+    if ((int)blockIdx.x < inlet_blocks) {
+        const int j = (int)blockIdx.x * NODES_PER_BLOCK + g;
+        if (j < a.n) inlet_eq(a, j, q);
         return;
     }
-    const Cell c = cell_at(a.g, b.x, b.y, b.z);
-    R d[Q];
-    int pl[Q];
-    uint32_t ix[Q];
-    load_node(a, c, d, pl, ix);
-    interp_outlet(d, b, a.pub_post, a.K, a.cs, a.crev20 != 0);
-    store_node(a, d, pl, ix);
+    const int j = ((int)blockIdx.x - inlet_blocks) * NODES_PER_BLOCK + g;
+    NodeDev b;
+    b.kind = -1;
+    if (j < n_outl) b = outl[j];
+    const bool act = b.kind == LBM_BC_OUTLET_INTERPOLATED && q < Q;
+    const bool crev20 = a.crev20 != 0;
+    typename ST::T* plane = nullptr;
+    uint32_t ix = 0;
+    R v = R(0);
+    if (act) {
+        int pl;
+        read_slot(cell_at(a.g, b.x, b.y, b.z), q, a.odd != 0, pl, ix);
+        plane = a.p[0] + (size_t)pl * (size_t)(a.p[1] - a.p[0]);
+        v = ST::load(plane, ix, a.rest[WCLASS[q]]);
+    }
+    sh[g][q] = v;
+    __syncthreads();
+    const bool blend = act && b.s1 != -2;
+    if (act) {
+        // the irregular node's copies d[vel] = d[crev vel], made in turn for vel
+        // in the mask: follow population q back to the value it ends up with
+        const uint32_t mask = (uint32_t)b.partner;
+        int from = q, turn = Q;
+        while (from < turn && ((mask >> from) & 1u)) {
+            turn = from;
+            from = crev_of(from, crev20);
+        }
+        v = sh[g][from];
+        const float nc = b.nx * (float)CX[q] + b.ny * (float)CY[q] + b.nz * (float)CZ[q];
+        if (blend && nc < 0.0f) {
+            const R up = b.s1 >= 0 ? a.pub_post[(size_t)b.s1 * Q + q] : R(0);
+            v = a.cs * up + (R(1) - a.cs) * a.pub_post[(size_t)b.s0 * Q + q];
+        }
+    }
+    __syncthreads();
+    sh[g][q] = v;
+    __syncthreads();
+    if (blend) {
+        R rho, ux, uy, uz;
+        outlet_moments<R>(sh[g], b.rho, rho, ux, uy, uz);
+        v = outlet_reset(a.K, q, v, ux, uy, uz, rho);
+    }
+    if (act) ST::store(plane, ix, v, a.rest[WCLASS[q]]);
 }
 
 // Periodic::periodic (Periodic.h:43-138): populations with n.c < 0 are
