@@ -26,7 +26,8 @@ struct lbm_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     size_t N = 0;              // padded cells
     size_t NP = 0;             // population plane stride: N up to a whole cache line
-    bool rows_aligned = true;  // rows start on a cache line
+    bool turn = false;         // odd steps take the tiles from the last to the first
+    bool nt_even = false, nt_odd = false;   // the step takes the streaming hint
     size_t NU = 0;             // caller's cells
     size_t elem = 0;           // bytes per stored population
     size_t rbytes = 0;         // bytes per arithmetic value

@@ -500,6 +500,50 @@ static int pick_bx_log2(int nx, bool flagged)
     return best;
 }
 
+// Streaming hint and tile order by the bytes of the populations.  The 256 MiB
+// cache in front of the HBM holds a smaller lattice from step to step, if no hint
+// sends its lines past it.  Of a larger one a sweep in the same order finds
+// nothing there again; an odd step that starts with the tiles the even step ended
+// with finds the last 256 MiB, less what the hint keeps out.  Measured, us a step
+// (none / even steps hinted / both hinted / in turn / in turn, odd steps hinted):
+//   box f32 128^3, 216 MiB        68 /  72 /  77 /  69 /  73
+//   box f32 160^3, 422            182 / 157 / 154 / 150 / 155
+//   box f32 192^3, 729            297 / 271 / 266 / 262 / 258
+//   box f32 256^3, 1728           680 / 639 / 628 / 667 / 641
+//   box f64 176x160x160, 928          / 360 / 350 / 355 / 348
+//   box f16 192^3, 364            152 / 136 / 138 / 131 / 135
+//   box f16 256^3, 864                / 333 / 342 / 323 / 332
+//   box f32 150x150x113, 262      110 /  94 / 100 / 100 /  95   (rows off the lines)
+//   box f32 203x160x131, 438      193 / 167 / 170 / 154 / 162   (rows off the lines)
+//   cavity f32 130x98x114, 191     62 /  71 /  74 /  60 /  66
+//   cavity f32 162x130x130, 344   155 / 137 / 134 / 145 / 137
+//   cavity f32 160^3, 412         216 / 203 / 192 / 175 / 171
+//   duct f32 200x128x128, 378     205 / 176 / 168 / 166 / 164
+//   duct f32 384x192x160, 1316        / 588 / 566 / 574 / 568
+//   duct f16 210x101x92, 123       66 /  83 /  85 /  66 /  77
+//   duct f16 512x160x128, 617         / 284 / 277 / 290 / 284
+static void pick_cache_use(lbm_ctx* c, size_t bytes, bool rows_aligned)
+{
+    const size_t MiB = (size_t)1 << 20;
+    const bool wide = c->elem >= 4;
+    c->turn = c->nt_even = c->nt_odd = false;
+    if (bytes <= 256 * MiB) return;
+    if (c->flags_needed) {
+        c->turn = wide && bytes > 352 * MiB && bytes <= 1024 * MiB;
+        c->nt_even = !c->turn;
+        c->nt_odd = true;
+    } else if (!wide) {
+        c->turn = true;
+    } else if (!rows_aligned) {
+        c->turn = bytes > 320 * MiB;
+        c->nt_even = !c->turn;
+    } else {
+        c->turn = bytes <= 1024 * MiB;
+        c->nt_even = !c->turn;
+        c->nt_odd = bytes > 512 * MiB;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
@@ -709,9 +753,10 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     c->g.tz0 = L.pz + lo[2];
     c->g.tex = ex;
     c->g.tey = ey;
-    c->rows_aligned = (size_t)L.nx * elem % 128 == 0;
+    const bool rows_aligned = (size_t)L.nx * elem % 128 == 0;
+    pick_cache_use(c, NP * elem * Q, rows_aligned);
     // consecutive cells where the rows leave lanes idle or start inside a line
-    c->g.flat = !P.flags_needed && (ex % (1 << bxl) != 0 || ey % c->g.by != 0 || !c->rows_aligned);
+    c->g.flat = !P.flags_needed && (ex % (1 << bxl) != 0 || ey % c->g.by != 0 || !rows_aligned);
     c->g.rnx = (uint32_t)((1ull << 32) / (uint64_t)L.nx);
     c->g.rny = (uint32_t)((1ull << 32) / (uint64_t)L.ny);
     if (c->g.flat) c->g.ntiles = (int)blocks_for(NU);

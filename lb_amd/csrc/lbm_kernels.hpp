@@ -77,6 +77,7 @@ struct Geo {
     int bx_log2, by;    // tile: (1 << bx_log2) x by cells, 256 threads
     int ntx, nty;       // tiles along x and y
     int ntiles;
+    int back;           // this step takes the tiles from the last to the first
     int wx, wy, wz;     // index wrap per axis
     int tx0, ty0, tz0;  // padded coordinates of the first tile: the box of non-solid cells
     int tex, tey;       // its extents along x and y
@@ -304,19 +305,26 @@ __device__ __forceinline__ uint32_t div_small(uint32_t n, uint32_t d, uint32_t r
     return q;
 }
 
+// This workgroup's place in the order of the tiles.
+__device__ __forceinline__ uint32_t tile_number(const Geo& g)
+{
+    return g.back ? (uint32_t)g.ntiles - 1u - blockIdx.x : blockIdx.x;
+}
+
 template <bool FLAGS>
 __device__ __forceinline__ Cell cell_of(const Geo& g)
 {
     Cell c;
+    const uint32_t b = tile_number(g);
     if (!FLAGS && g.flat) {
-        c.i = blockIdx.x * (uint32_t)TPB + threadIdx.x;
+        c.i = b * (uint32_t)TPB + threadIdx.x;
         c.inside = c.i < (uint32_t)g.nx * (uint32_t)g.ny * (uint32_t)g.nz;
         uint32_t x, y;
         c.z = (int)div_small(div_small(c.i, (uint32_t)g.nx, g.rnx, x), (uint32_t)g.ny, g.rny, y);
         c.x = (int)x;
         c.y = (int)y;
     } else {
-        const int t = tile_of_block(g, (int)blockIdx.x);
+        const int t = tile_of_block(g, (int)b);
         const int tx = t % g.ntx;
         const int rem = t / g.ntx;
         const int ty = rem % g.nty;
@@ -357,8 +365,8 @@ __device__ __forceinline__ void read_slot(const Cell& c, int q, bool odd, int& p
 
 // A wave's access to population q covers whole cache lines when it is not
 // shifted along x: every access of the even step, and on the odd step the
-// directions with c_x = 0, if rows start on a line (the odd step's kernel is
-// compiled for both, NT = false where they do not).
+// directions with c_x = 0, if rows start on a line (the kernels are compiled with
+// the streaming hint and without, pick_cache_use chooses).
 __host__ __device__ constexpr bool line_aligned(bool odd, int q) { return !odd || CX[q] == 0; }
 __host__ __device__ constexpr int read_plane(bool odd, int q) { return odd ? OPP[q] : q; }
 __device__ __forceinline__ uint32_t read_index(const Cell& c, bool odd, int q) { return odd ? nb(c, OPP[q]) : c.i; }
@@ -495,7 +503,7 @@ __device__ __forceinline__ void moment_add(double* avg, size_t nu, size_t iu, do
 // collision: f = pre-collision populations, P = post-collision populations.
 // (k_step keeps its own inline copy of this code: passing the population
 // arrays through a helper raised its register count from 48-64 to > 100.)
-template <class ST, bool ODD, bool FLAGS>
+template <class ST, bool ODD, bool FLAGS, bool NT>
 __device__ __forceinline__ void stream_cell(const StepArgs<ST>& a, const Cell& c, uint8_t cls, int bi, bool inlet,
                                             typename ST::R (&P)[Q],
                                             typename ST::R rho, typename ST::R ux, typename ST::R uy,
@@ -557,7 +565,7 @@ __device__ __forceinline__ void stream_cell(const StepArgs<ST>& a, const Cell& c
 #pragma unroll
     for (int q = 0; q < Q; ++q)
         if (line_aligned(ODD, q) && !((Kk >> q) & 1u))
-            store_out<ST, ODD, true>(a.p, a.rest, c, q, P[q], hsr);
+            store_out<ST, ODD, NT>(a.p, a.rest, c, q, P[q], hsr);
 #pragma unroll
     for (int q = 0; q < Q; ++q)
         if (!line_aligned(ODD, q) && !((Kk >> q) & 1u))
@@ -583,7 +591,7 @@ __device__ __forceinline__ void step_cells(const StepArgs<ST>& a)
 // waves: they need 64 VGPRs with the cumulant operators (8 waves), and a hint for
 // 7 made BGK and the 2017 operators spill 650 bytes a lane (210 x 101 x 92 duct,
 // FP16, 2017: 140 -> 95 us a step without it).
-template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC = false, bool INL = false, bool NT = true>
+template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC, bool INL, bool NT>
 __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
 {
     if constexpr (sizeof(typename ST::T) == 4) {
@@ -638,7 +646,7 @@ __device__ __forceinline__ void closure_prep(const typename ST::R* f, bool first
 // lane takes part, cells without a collision feed zeros); phase 3 collides
 // with omega from the network's coefficient -- or from the Smagorinsky
 // formula when a feature leaves the training envelope -- and streams.
-template <class ST, int COLL, bool ODD, bool FLAGS>
+template <class ST, int COLL, bool ODD, bool FLAGS, bool NT>
 __global__ __launch_bounds__(TPB) void k_step_mlp(MlpStepArgs<ST> ma)
 {
     const StepArgs<ST>& a = ma.s;
@@ -667,7 +675,7 @@ __global__ __launch_bounds__(TPB) void k_step_mlp(MlpStepArgs<ST> ma)
 #pragma unroll
             for (int q = 0; q < Q; ++q) f[q] = a.inl_state[(size_t)bi * Q + q];
         } else {
-            load_pop<ST, ODD>(a.p, a.rest, c, f);
+            load_pop<ST, ODD, NT>(a.p, a.rest, c, f);
         }
         closure_prep<ST>(f, a.first != 0, a.macro, (size_t)a.g.n, c.i, a.tau, a.cles, L, cp);
         if (cp.env) {
@@ -693,7 +701,7 @@ __global__ __launch_bounds__(TPB) void k_step_mlp(MlpStepArgs<ST> ma)
         Cell cs = c;
         __asm__ volatile("" : "+v"(cs.i), "+v"(cs.dxm), "+v"(cs.dxp), "+v"(cs.dym), "+v"(cs.dyp), "+v"(cs.dzm),
                          "+v"(cs.dzp));
-        stream_cell<ST, ODD, FLAGS>(a, cs, cls, bi, inlet, P, cp.rho, cp.ux, cp.uy, cp.uz);
+        stream_cell<ST, ODD, FLAGS, NT>(a, cs, cls, bi, inlet, P, cp.rho, cp.ux, cp.uy, cp.uz);
     }
 }
 

@@ -6,6 +6,25 @@
 #error "LBM_STORE names the storage policy of this translation unit"
 #endif
 
+// One step of either parity, with the streaming hint (nt) or without.
+template <class ST, int COLL, bool LIT, bool FLAGS, bool CC, bool INL>
+static void launch_step(bool odd, bool nt, dim3 grid, hipStream_t s, const StepArgs<ST>& a)
+{
+    if (odd && nt) k_step<ST, COLL, LIT, true, FLAGS, CC, INL, true><<<grid, TPB, 0, s>>>(a);
+    else if (odd) k_step<ST, COLL, LIT, true, FLAGS, CC, INL, false><<<grid, TPB, 0, s>>>(a);
+    else if (nt) k_step<ST, COLL, LIT, false, FLAGS, CC, INL, true><<<grid, TPB, 0, s>>>(a);
+    else k_step<ST, COLL, LIT, false, FLAGS, CC, INL, false><<<grid, TPB, 0, s>>>(a);
+}
+
+template <class ST, int COLL, bool FLAGS>
+static void launch_mlp(bool odd, bool nt, dim3 grid, hipStream_t s, const MlpStepArgs<ST>& a)
+{
+    if (odd && nt) k_step_mlp<ST, COLL, true, FLAGS, true><<<grid, TPB, 0, s>>>(a);
+    else if (odd) k_step_mlp<ST, COLL, true, FLAGS, false><<<grid, TPB, 0, s>>>(a);
+    else if (nt) k_step_mlp<ST, COLL, false, FLAGS, true><<<grid, TPB, 0, s>>>(a);
+    else k_step_mlp<ST, COLL, false, FLAGS, false><<<grid, TPB, 0, s>>>(a);
+}
+
 template <class ST, int COLL, bool LIT>
 static lbm_status launch_steps(lbm_ctx* c, int nsteps)
 {
@@ -44,7 +63,7 @@ static lbm_status launch_steps(lbm_ctx* c, int nsteps)
     }
     const bool patches = (c->n_upd && !c->inl_deferred) || c->n_eq || (c->n_outlet && !c->outl_deferred) ||
                          c->n_ghost;
-    const dim3 grid((unsigned)c->g.ntiles), block(TPB);
+    const dim3 grid((unsigned)c->g.ntiles);
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     for (int s = 0; s < nsteps; ++s) {
         a.first = c->first ? 1 : 0;
@@ -63,41 +82,24 @@ static lbm_status launch_steps(lbm_ctx* c, int nsteps)
         a.inl_pending = c->inl_pending ? 1 : 0;
         if constexpr (ST::sr) a.seed = step_seed((uint64_t)c->steps);
         const bool odd = (c->steps & 1) != 0;
+        a.g.back = odd && c->turn;
+        const bool nt = odd ? c->nt_odd : c->nt_even;
         if constexpr (sizeof(R) == 4 && !LIT && COLL <= LBM_COLLISION_CUM2015) {
             if (mlp && c->cl_count % c->cl_every == 0) {
                 // network evaluated in this step; coefficients kept for the next ones
                 ma.s = a;
-                if (c->flags_needed) {
-                    if (odd) k_step_mlp<ST, COLL, true, true><<<grid, block, 0, c->stream>>>(ma);
-                    else k_step_mlp<ST, COLL, false, true><<<grid, block, 0, c->stream>>>(ma);
-                } else {
-                    if (odd) k_step_mlp<ST, COLL, true, false><<<grid, block, 0, c->stream>>>(ma);
-                    else k_step_mlp<ST, COLL, false, false><<<grid, block, 0, c->stream>>>(ma);
-                }
+                if (c->flags_needed) launch_mlp<ST, COLL, true>(odd, nt, grid, c->stream, ma);
+                else launch_mlp<ST, COLL, false>(odd, nt, grid, c->stream, ma);
             } else if (mlp) {
-                if (c->flags_needed) {
-                    if (odd) k_step<ST, COLL, false, true, true, true><<<grid, block, 0, c->stream>>>(a);
-                    else k_step<ST, COLL, false, false, true, true><<<grid, block, 0, c->stream>>>(a);
-                } else {
-                    if (odd && !c->rows_aligned) k_step<ST, COLL, false, true, false, true, false, false><<<grid, block, 0, c->stream>>>(a);
-                    else if (odd) k_step<ST, COLL, false, true, false, true><<<grid, block, 0, c->stream>>>(a);
-                    else k_step<ST, COLL, false, false, false, true><<<grid, block, 0, c->stream>>>(a);
-                }
+                if (c->flags_needed) launch_step<ST, COLL, false, true, true, false>(odd, nt, grid, c->stream, a);
+                else launch_step<ST, COLL, false, false, true, false>(odd, nt, grid, c->stream, a);
             }
             if (mlp) c->cl_count++;
         }
         if (!mlp) {
-            if (c->flags_needed && c->inl_deferred) {
-                if (odd) k_step<ST, COLL, LIT, true, true, false, true><<<grid, block, 0, c->stream>>>(a);
-                else k_step<ST, COLL, LIT, false, true, false, true><<<grid, block, 0, c->stream>>>(a);
-            } else if (c->flags_needed) {
-                if (odd) k_step<ST, COLL, LIT, true, true><<<grid, block, 0, c->stream>>>(a);
-                else k_step<ST, COLL, LIT, false, true><<<grid, block, 0, c->stream>>>(a);
-            } else {
-                if (odd && !c->rows_aligned) k_step<ST, COLL, LIT, true, false, false, false, false><<<grid, block, 0, c->stream>>>(a);
-                else if (odd) k_step<ST, COLL, LIT, true, false><<<grid, block, 0, c->stream>>>(a);
-                else k_step<ST, COLL, LIT, false, false><<<grid, block, 0, c->stream>>>(a);
-            }
+            if (!c->flags_needed) launch_step<ST, COLL, LIT, false, false, false>(odd, nt, grid, c->stream, a);
+            else if (c->inl_deferred) launch_step<ST, COLL, LIT, true, false, true>(odd, nt, grid, c->stream, a);
+            else launch_step<ST, COLL, LIT, true, false, false>(odd, nt, grid, c->stream, a);
         }
         HIPCHK(hipGetLastError());
         if (patches) {

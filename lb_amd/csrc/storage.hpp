@@ -35,10 +35,10 @@ __device__ __forceinline__ T& at(T* p, uint32_t i)
 // Plain or non-temporal (streaming) access to element i, chosen at compile
 // time (a run-time choice between two accesses to one address lets the
 // compiler merge them and drop the hint).  The collide-stream step streams
-// every population once per step; where a wave's access covers whole cache
-// lines (every access of the even step, and the directions without an x
-// component on the odd step), the streaming hint keeps those lines from
-// displacing the partial lines that neighbouring tiles share.
+// every population once per step; on lattices that the caches do not hold, where
+// a wave's access covers whole cache lines (every access of the even step, and the
+// directions without an x component on the odd step), the streaming hint keeps
+// those lines from displacing the partial lines that neighbouring tiles share.
 template <bool NT, class T>
 __device__ __forceinline__ T ld(const T* p, uint32_t i)
 {
