@@ -946,7 +946,7 @@ lbm_status lbm_moment_avg(lbm_ctx* c, double* rho, double* ux, double* uy, doubl
     double* outs[4] = {rho, ux, uy, uz};
     // momentAvg (MomentTimeAvg.h:47-77): the sums divided by the counter
     const double n = (double)c->avg_count;
-    if (ring_ready(c)) return read_planes(c, c->avg, outs, 4, n);
+    if (ring_ready(c, 4)) return read_planes(c, c->avg, outs, 4, n);
     for (int k = 0; k < 4; ++k)
         if (outs[k])
             HIPCHK(hipMemcpyAsync(outs[k], c->avg + k * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost,
@@ -1026,7 +1026,7 @@ lbm_status lbm_get_macroscopic(lbm_ctx* c, double* rho, double* ux, double* uy, 
     lbm_status st = lbm_sync(c);
     if (st != LBM_OK && st != LBM_E_NAN) return st;
     double* outs[4] = {rho, ux, uy, uz};
-    if (ring_ready(c))
+    if (ring_ready(c, 4))
         return with_storage(c, [&](auto stv) -> lbm_status {
             using ST = decltype(stv);
             using R = typename ST::R;
@@ -1131,7 +1131,7 @@ lbm_status lbm_get_omega(lbm_ctx* c, double* omega)
         st = run_macro(c);
     }
     if (st != LBM_OK) return st;
-    if (ring_ready(c)) return read_planes(c, c->stage + 4 * c->NU, &omega, 1);
+    if (ring_ready(c, 1)) return read_planes(c, c->stage + 4 * c->NU, &omega, 1);
     HIPCHK(hipMemcpyAsync(omega, c->stage + 4 * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1205,7 +1205,7 @@ lbm_status lbm_get_population(lbm_ctx* c, int32_t q, double* f)
         return LBM_OK;
     });
     if (st != LBM_OK) return st;
-    if (ring_ready(c)) return read_planes(c, c->stage, &f, 1);
+    if (ring_ready(c, 1)) return read_planes(c, c->stage, &f, 1);
     HIPCHK(hipMemcpyAsync(f, c->stage, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1228,7 +1228,7 @@ lbm_status lbm_get_populations(lbm_ctx* c, double* f)
         });
         if (st != LBM_OK) return st;
         double* fq = f + (size_t)q * c->NU;
-        if (ring_ready(c)) {
+        if (ring_ready(c, 1)) {
             st = read_planes(c, c->stage, &fq, 1);
             if (st != LBM_OK) return st;
             continue;

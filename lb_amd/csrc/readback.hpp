@@ -17,9 +17,18 @@
 
 #include "context.hpp"
 
-// The ring, allocated by the first read of a context (false: no pinned memory).
-static inline bool ring_ready(lbm_ctx* c)
+// True where np planes go through the ring, which the first such read of a
+// context allocates (false too if there is no pinned memory): where one slot holds
+// them, which takes no other thread, and from 96 MiB on.  Between, the copies into
+// the caller's memory stay: a caller's own thread pool that spins on every CPU
+// between its uses (OpenMP's default) was held up for some 10 ms after the ring's
+// threads had run.  With such a pool, a pass of the 130x98x114 cavity (46 MB)
+// took 18.4 ms without the ring and 18.8 with it, the 203x97x131 box (82 MB) 14 and
+// 25; the 256^3 box (537 MB) 251 and 227, the 160x144x160 FP64 box (118 MB) 52 and 47.
+static inline bool ring_ready(lbm_ctx* c, int np)
 {
+    const size_t bytes = (size_t)np * c->NU * sizeof(double);
+    if (bytes > RB_SLOT && bytes < RB_MANY) return false;
     if (c->rb_host) return true;
     for (hipEvent_t& e : c->rb_ev)
         if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
