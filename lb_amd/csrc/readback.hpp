@@ -23,21 +23,22 @@
 // the caller's memory stay: a caller's own thread pool that spins on every CPU
 // between its uses (OpenMP's default) was held up for some 10 ms after the ring's
 // threads had run.  With such a pool, a pass of the 130x98x114 cavity (46 MB)
-// took 18.4 ms without the ring and 18.8 with it, the 203x97x131 box (82 MB) 14 and
-// 25; the 256^3 box (537 MB) 251 and 227, the 160x144x160 FP64 box (118 MB) 52 and 47.
+// took 17.8 ms without the ring and 20.5 with it, the 203x97x131 box (82 MB) 16.3 and
+// 24.6; the 256^3 box (537 MB) 251 and 227, the 160x144x160 FP64 box (118 MB) 52.5 and
+// 47.1.
 static inline bool ring_ready(lbm_ctx* c, int np)
 {
     const size_t bytes = (size_t)np * c->NU * sizeof(double);
     if (bytes > RB_SLOT && bytes < RB_MANY) return false;
     if (c->rb_host) return true;
-    for (hipEvent_t& e : c->rb_ev)
-        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            e = nullptr;
-            return false;
-        }
     // no more slots than five FP64 planes fill
     c->rb_slots = (int)std::min<size_t>(RB_SLOTS, (5 * c->NU * sizeof(double) + RB_SLOT - 1) / RB_SLOT);
+    for (int k = 0; k < c->rb_slots; ++k)
+        if (!c->rb_ev[k] && hipEventCreateWithFlags(&c->rb_ev[k], hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            c->rb_ev[k] = nullptr;
+            return false;
+        }
     if (hipHostMalloc((void**)&c->rb_host, RB_SLOT * c->rb_slots, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         c->rb_host = nullptr;
