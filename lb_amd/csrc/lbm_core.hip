@@ -760,6 +760,8 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     c->g.rnx = (uint32_t)((1ull << 32) / (uint64_t)L.nx);
     c->g.rny = (uint32_t)((1ull << 32) / (uint64_t)L.ny);
     if (c->g.flat) c->g.ntiles = (int)blocks_for(NU);
+    c->g.hash_dx = L.w[0] ? 0 : line - L.px;
+    c->g.hash_nx = L.w[0] ? L.nx : (line + L.ux + 1 + line - 1) / line * line;
     c->g.wx = L.w[0];
     c->g.wy = L.w[1];
     c->g.wz = L.w[2];

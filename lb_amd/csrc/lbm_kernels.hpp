@@ -83,6 +83,7 @@ struct Geo {
     int tex, tey;       // its extents along x and y
     int flat;           // no metadata: tile = 256 consecutive cells of the lattice
     uint32_t rnx, rny;  // floor(2^32 / nx), floor(2^32 / ny)
+    int hash_dx, hash_nx;   // sr_index: shift along x, row pitch
 };
 
 // Boundary-node record on the device (padded coordinates).  Publish slots
@@ -247,6 +248,17 @@ __device__ __forceinline__ void set_deltas(const Geo& g, Cell& c)
     c.dyp = (c.y < g.ny - 1 || !g.wy) ? sy : -(g.ny - 1) * sy;
     c.dzm = (c.z > 0 || !g.wz) ? -sz : (g.nz - 1) * sz;
     c.dzp = (c.z < g.nz - 1 || !g.wz) ? sz : -(g.nz - 1) * sz;
+}
+
+// The cell's number for the random bits of the stochastic-rounding stores.  It
+// depends on the caller's extents and the element size alone, so that a run draws
+// the same bits wherever the layout puts its rows: the index in rows that hold a
+// cache line of halo before the caller's first cell and one cell or more after
+// the last (without index wrap in x), or none (with it, where it is c.i).
+template <bool FLAGS>
+__device__ __forceinline__ uint32_t sr_index(const Geo& g, const Cell& c)
+{
+    return FLAGS ? (uint32_t)(c.x + g.hash_dx + g.hash_nx * (c.y + g.ny * c.z)) : c.i;
 }
 
 __device__ __forceinline__ Cell cell_at(const Geo& g, int x, int y, int z)
@@ -510,7 +522,7 @@ __device__ __forceinline__ void stream_cell(const StepArgs<ST>& a, const Cell& c
                                             typename ST::R uz)
 {
     using R = typename ST::R;
-    const uint32_t hsr = ST::sr ? sr_hash(c.i, a.seed) : 0u;
+    const uint32_t hsr = ST::sr ? sr_hash(sr_index<FLAGS>(a.g, c), a.seed) : 0u;
     // node word of a boundary cell (0 for plain fluid): skip masks and walls
     const uint64_t nw = (FLAGS && cls != CL_FLUID) ? a.node[c.i] : 0ull;
     const uint32_t S = (uint32_t)(nw & MASK27);

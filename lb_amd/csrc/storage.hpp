@@ -193,7 +193,7 @@ struct StoreBF16DevSR : StoreBF16Dev {
 
 // Random bits of one cell and step for the stochastic-rounding stores: the
 // "lowbias32" integer hash (C. Wellons, hash-prospector; xor-shift-multiply
-// rounds) of the cell index xor the step seed; population q uses
+// rounds) of the cell's number (sr_index) xor the step seed; population q uses
 // h + q * 0x9E3779B9 (a Weyl sequence, whose high bits the conversions read).
 __device__ __forceinline__ uint32_t sr_hash(uint32_t i, uint32_t seed)
 {
