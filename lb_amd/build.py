@@ -95,13 +95,11 @@ def build_oracle():
 
 def build_tests():
     nat = os.path.join(ROOT, "tests", "native")
-    src = os.path.join(nat, "collide_host.cpp")
-    if not os.path.exists(src):
-        return None
-    out = os.path.join(nat, "libcollide_host.so")
-    _run([CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-fno-fast-math",
-          f"-I{CSRC}", f"-I{os.path.join(ROOT, 'include')}", "-o", out, src])
-    return out
+    for name in ("collide_host", "collide_fp64_host"):
+        src = os.path.join(nat, name + ".cpp")
+        if os.path.exists(src):
+            _run([CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-fno-fast-math",
+                  f"-I{CSRC}", f"-I{os.path.join(ROOT, 'include')}", "-o", os.path.join(nat, f"lib{name}.so"), src])
 
 
 def build_all():

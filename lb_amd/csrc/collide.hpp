@@ -95,49 +95,6 @@ LBM_HD R fma_r(R a, R b, R c)
     return std::fma(a, b, c);
 }
 
-// Reciprocal of a positive normal number (a density, a relaxation time): the
-// hardware FP32 reciprocal and one Newton step in fused multiply-adds, which
-// leave the error at the half ulp of the last rounding, in 3 instructions
-// where the IEEE quotient's scaling and fix-up take 11.
-template <class R>
-LBM_HD R rcp_nr(R x)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (sizeof(R) == 4) {
-        const R r = __builtin_amdgcn_rcpf(x);
-        return fma_r(fma_r(-x, r, R(1)), r, r);
-    }
-#endif
-    return R(1) / x;
-}
-
-// Square root of a positive normal number: the hardware inverse square root
-// and one correction, exact to the half ulp of the last rounding (5
-// instructions; the IEEE square root takes 16).
-template <class R>
-LBM_HD R sqrt_nr(R x)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (sizeof(R) == 4) {
-        const R y = __builtin_amdgcn_rsqf(x);
-        const R s = x * y;
-        return fma_r(fma_r(-s, s, x), R(0.5) * y, s);
-    }
-#endif
-    return std::sqrt(x);
-}
-
-// Square root, 0 included: the hardware FP32 instruction (within 1 ulp) on
-// the device, correctly rounded otherwise.
-template <class R>
-LBM_HD R fsqrt(R x)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (sizeof(R) == 4) return __builtin_amdgcn_sqrtf(x);
-#endif
-    return std::sqrt(x);
-}
-
 // Base-10 logarithm for the closure features: the hardware log2 (within
 // 1 ulp for normal inputs) times log10(2) on the device in FP32, the library
 // function otherwise.
@@ -826,8 +783,7 @@ LBM_HD void cum2017_fast(const Consts<R>& K, const R* fin, const Cen2<R>& c, R m
 }
 
 // ---------------------------------------------------------------------------
-// The same operators in fewer operations, for the storage formats whose
-// results may be rounded differently (see Ops below).
+// The same operators in fewer operations, for FP64 storage (see Ops below).
 // ---------------------------------------------------------------------------
 
 // Sum (x - ux)^2 f = mxx - ux (jx + k100) and sum (x - ux)(y - uy) f =
@@ -835,7 +791,8 @@ LBM_HD void cum2017_fast(const Consts<R>& K, const R* fin, const Cen2<R>& c, R m
 // the first step after an initialisation): 15 multiply-adds and three sums
 // where the written-out squares take 57 operations, and fewer roundings.
 // Fused multiply-adds are written out and contraction is off, here and in the
-// functions below: every kernel that forms the rate gets the same bits.
+// other functions of the rate: the step and the read-back of omega form the same
+// bits.
 template <class R>
 LBM_HD Cen2<R> central2_fused(const Raw2<R>& r, R ux, R uy, R uz)
 {
@@ -856,9 +813,6 @@ LBM_HD Cen2<R> central2_fused(const Raw2<R>& r, R ux, R uy, R uz)
 // |Pi_neq| / rho: see omega_les_fast.  For D3Q27 the second-order equilibrium moments are
 // rho*(u u + I/3), so Pi_neq = central second moments - rho/3 I (the
 // reference builds the same tensor with a 27-term loop, OmegaLES.h:84-101).
-// The norm's argument carries the cancellation error of that difference
-// (about 1e-3 relative in FP32), so the hardware square root (within 1 ulp)
-// adds nothing to it.
 template <class R>
 LBM_HD R pin_over_rho_fused(const Cen2<R>& c, R rho)
 {
@@ -867,7 +821,7 @@ LBM_HD R pin_over_rho_fused(const Cen2<R>& c, R rho)
             pzz = fma_r(R(-1.0 / 3.0), rho, c.kzz);
     const R off = fma_r(c.kxy, c.kxy, fma_r(c.kxz, c.kxz, c.kyz * c.kyz));
     const R n2 = fma_r(R(2), off, fma_r(pxx, pxx, fma_r(pyy, pyy, pzz * pzz)));
-    return fsqrt(n2) * rcp_nr(rho);
+    return std::sqrt(n2) * (R(1) / rho);   // the step's own 1 / rho
 }
 
 // Relaxation time from a coefficient C: the reference's formula
@@ -876,18 +830,17 @@ template <class R>
 LBM_HD R tau_from_coefficient_fused(R C, R pin_rho, R tau0)
 {
     LBM_FP_STRICT
-    return fma_r(R(0.5), sqrt_nr(fma_r(R(18) * C, pin_rho, tau0 * tau0)), R(0.5) * tau0);
+    return fma_r(R(0.5), std::sqrt(fma_r(R(18) * C, pin_rho, tau0 * tau0)), R(0.5) * tau0);
 }
 
 // Rate from a closure coefficient C.
 template <class R>
 LBM_HD R omega_from_coefficient_fused(R C, R pin_rho, R tau0)
 {
-    return rcp_nr(tau_from_coefficient_fused(C, pin_rho, tau0));
+    return R(1) / tau_from_coefficient_fused(C, pin_rho, tau0);
 }
 
-// Smagorinsky rate from the non-equilibrium stress; the learned closure's
-// fallback evaluates this same formula in another kernel.
+// Smagorinsky rate from the non-equilibrium stress.
 template <class R>
 LBM_HD R omega_les_fused(const Cen2<R>& c, R rho, R tau, R cles)
 {
@@ -971,9 +924,8 @@ LBM_HD void inv_yz(R* X, R uy, R uz, R* f)
 // fields the step uses (equal to the moments of f except on the first step
 // after an equilibrium initialisation).  Writes post-collision populations.
 //
-// What bounds it is the number of vector instructions: 16-bit storage moves
-// so few bytes that the step waits for them, and FP32 does once two steps
-// share one pass over memory.  With every cumulant of order >= 3 zero the
+// What bounds it where a lattice fits the caches or has boundaries is the number of
+// vector instructions.  With every cumulant of order >= 3 zero the
 // state is a Gaussian, whose moments of order 4 and 6 follow from those of
 // order 2 (Eq. G2015 81-84 with those cumulants dropped): in
 // x = s200, ..., over rho, s220 = rho (ab + 2 d^2), s211 = rho (a f + 2 d e)
@@ -985,7 +937,7 @@ template <class R>
 LBM_HD void cum2015_fused(const Consts<R>& K, const Cen2<R>& c, R m0, R rho, R ux, R uy, R uz, R omg, R* f)
 {
     LBM_FP_STRICT
-    const R ir = rcp_nr(rho);
+    const R ir = R(1) / rho;
     const R C200 = c.kxx, C020 = c.kyy, C002 = c.kzz;
     const R d1 = C200 - C020, d2 = C200 - C002;
     const R hw = R(0.5) * omg * ir, hw3 = R(3) * hw;
@@ -1097,7 +1049,7 @@ LBM_HD void cum2017_fused(const Consts<R>& K, const R* fin, const Cen2<R>& c, R 
     const R C210 = third(t.m210, uy, r.mxx, ux, c.kxy, c.k010), C012 = third(t.m012, uy, r.mzz, uz, c.kyz, c.k010);
     const R C201 = third(t.m201, uz, r.mxx, ux, c.kxz, c.k001), C021 = third(t.m021, uz, r.myy, uy, c.kyz, c.k001);
     const R C111 = fma_r(-ux, c.kyz, fma_r(-uy, fma_r(-uz, r.jx, r.mxz), fma_r(-uz, r.mxy, t.m111)));
-    const R ir = rcp_nr(rho);
+    const R ir = R(1) / rho;
     const R C200 = c.kxx, C020 = c.kyy, C002 = c.kzz;
 
     // rates and limiters (Turbulent2017.h:240-291) with omega_2 = 1 substituted
@@ -1195,20 +1147,18 @@ LBM_HD void cum2017_fused(const Consts<R>& K, const R* fin, const Cen2<R>& c, R 
     inv_yz(X, uy, uz, f);
 }
 
-// Which of the two forms a kernel runs.  FP32 storage keeps the written-out
-// operation order: its results are compared with earlier ones at single
-// precision, and a uniform stream rounds alike in every cell, so that another
-// order drifts away from it by 1e-4 of a cross-stream velocity in 300 steps.
-// For 16-bit storage such differences vanish in the rounding of the stored
-// populations, and in FP64 they are 1e-15.
+// Which of the two forms a kernel runs: FP64 storage the one in fewer operations,
+// as its steps wait for their instructions on small lattices and on lattices with
+// boundaries (us a step, written out / fused: 64^3 box, 2017, 22.0 / 20.0; 66^3 cavity
+// 31.1 / 27.9; 150 x 77 x 92 duct, 2017, 122.5 / 113.7).  The two differ by roundings
+// of FP64; the fused form's error is no larger.  FP32 and 16-bit storage keep
+// the written-out operation order.  In FP32 a uniform stream rounds alike in every
+// cell, so that another order drifts away from it by 1e-4 of a cross-stream velocity
+// in 300 steps.  In 16 bits single flipped roundings of the stored populations grow
+// to another sample of the format's error within tens of steps: up to 1e-2 of a
+// velocity component in BF16.
 template <bool FUSED>
 struct Ops {
-    template <class R>
-    LBM_HD static R rcp(R x)
-    {
-        if constexpr (FUSED) return rcp_nr(x);
-        return R(1) / x;
-    }
     template <class R>
     LBM_HD static Cen2<R> cen2(const Raw2<R>& r, R ux, R uy, R uz)
     {

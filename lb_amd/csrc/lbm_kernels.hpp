@@ -600,9 +600,7 @@ __device__ __forceinline__ void step_cells(const StepArgs<ST>& a)
 // before its stores (107 VGPRs) and ran 2.9 % faster on the periodic 256^3
 // workload (cumulant 2017: 3.2 %), while the 16-bit steps ran 2.1-2.6 %
 // slower that way and FP64 0.5 %.  No launch bound holds the 16-bit steps to more
-// waves: they need 64 VGPRs with the cumulant operators (8 waves), and a hint for
-// 7 made BGK and the 2017 operators spill 650 bytes a lane (210 x 101 x 92 duct,
-// FP16, 2017: 140 -> 95 us a step without it).
+// waves: a hint for 7 made BGK and the 2017 operators spill 650 bytes a lane.
 template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC, bool INL, bool NT>
 __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
 {
@@ -630,7 +628,6 @@ __device__ __forceinline__ void closure_prep(const typename ST::R* f, bool first
                                              const MlpLds& L, ClosurePrep<ST>& o)
 {
     using R = typename ST::R;
-    using O = Ops<ST::fused>;
     const Raw2<R> r = raw_moments(f);
     o.m0 = r.m0;
     if (first) {
@@ -640,13 +637,13 @@ __device__ __forceinline__ void closure_prep(const typename ST::R* f, bool first
         o.uz = macro[3 * N + i];
     } else {
         o.rho = r.m0;
-        const R ir = O::rcp(o.rho);
+        const R ir = R(1) / o.rho;
         o.ux = r.jx * ir;
         o.uy = r.jy * ir;
         o.uz = r.jz * ir;
     }
-    o.ce = O::cen2(r, o.ux, o.uy, o.uz);
-    o.om_s = O::omega_les(o.ce, o.rho, tau, cles);
+    o.ce = central2(r, o.ux, o.uy, o.uz);
+    o.om_s = omega_les_fast(o.ce, o.rho, tau, cles);
     R om_unused;
     cell_features(o.ce, o.rho, tau, cles, o.x, o.pin, om_unused);
     o.env = mlp_normalise(L, o.x, o.xn);
@@ -701,7 +698,7 @@ __global__ __launch_bounds__(TPB) void k_step_mlp(MlpStepArgs<ST> ma)
         if (a.ccache) a.ccache[c.i] = cp.env ? mlp_coefficient(z, ma.mlp.c) : (float)a.cles;
         R P[Q];
         if (COLL == LBM_COLLISION_CUM2015) {
-            Ops<ST::fused>::cum2015(a.K, cp.ce, cp.m0, cp.rho, cp.ux, cp.uy, cp.uz, omega, P);
+            cum2015_fast(a.K, cp.ce, cp.m0, cp.rho, cp.ux, cp.uy, cp.uz, omega, P);
         } else {
 #pragma unroll
             for (int q = 0; q < Q; ++q) P[q] = f[q];
@@ -1209,7 +1206,7 @@ __device__ __forceinline__ void cell_macro(const AuxArgs<ST>& a, const Cell& c, 
             // the rate from the velocity as the step forms it (reciprocal, then products)
             R vx = ux, vy = uy, vz = uz;
             if (!a.first) {
-                const R ir = O::rcp(rho);
+                const R ir = R(1) / rho;
                 vx = r.jx * ir;
                 vy = r.jy * ir;
                 vz = r.jz * ir;

@@ -103,7 +103,7 @@ struct StoreF16Dev {
     using T = _Float16;
     using R = float;
     static constexpr bool dev = true;
-    static constexpr bool fused = true;
+    static constexpr bool fused = false;
     static constexpr bool sr = false;
     __device__ __forceinline__ static R load(const T* p, uint32_t i, R rest) { return (float)at(p, i) + rest; }
     __device__ __forceinline__ static void store(T* p, uint32_t i, R v, R rest) { at(p, i) = (_Float16)(v - rest); }
@@ -125,7 +125,7 @@ struct StoreBF16Dev {
     using T = uint16_t;
     using R = float;
     static constexpr bool dev = true;
-    static constexpr bool fused = true;
+    static constexpr bool fused = false;
     static constexpr bool sr = false;
     __device__ __forceinline__ static R load(const T* p, uint32_t i, R rest)
     {
