@@ -476,26 +476,23 @@ static lbm_status upload_macro(lbm_ctx* c, const double* rho, const double* ux, 
     return LBM_OK;
 }
 
-// Tile width 2^bxl along x.  Without metadata: the widest whose padding waste
-// stays under 15%, else the one with the least waste.  Boundary-aware steps: 256
-// where it wastes under 20%; otherwise 64, or 32 where that wastes at least 5%
-// less.  Measured, us a step: 128-wide cavity, FP32, 64: 86, 32: 88, 128: 96;
-// 64-wide cavity, FP64, 32: 30, 64: 31; 256-wide duct, FP32, 256: 212, 128: 228,
-// 32: 238, 64: 274; 210-wide duct, FP16, 256: 100, 128: 102, 32: 107, 64: 113.
-static int pick_bx_log2(int nx, bool flagged)
+// Tile width 2^bxl along x: the widest whose padding waste stays under 15%,
+// else the one with the least waste.  A line at 20% for boundary-aware steps, and 64
+// for what it refuses, lose: 210 x 101 x 92 duct, FP64, combined operator, 32 wide
+// 194 us a step, 256 wide 226; 128 x 100 x 90 duct, FP32, 128 wide 66, 64 wide 73;
+// 333 x 100 x 90 channel with index wrap in x, FP32, 128 wide 159, 32 wide 235.
+static int pick_bx_log2(int nx)
 {
-    auto util = [nx](int b) {
-        const int w = 1 << b;
-        return (double)nx / (double)(((nx + w - 1) / w) * w);
-    };
-    if (flagged) {
-        if (util(8) >= 0.8) return 8;
-        return util(5) >= util(6) + 0.05 ? 5 : 6;
-    }
     int best = 8;
+    double best_util = 0.0;
     for (int b = 8; b >= 5; --b) {
-        if (util(b) >= 0.85) return b;
-        if (util(b) > util(best)) best = b;
+        const int w = 1 << b;
+        const double util = (double)nx / (double)(((nx + w - 1) / w) * w);
+        if (util >= 0.85) return b;
+        if (util > best_util) {
+            best_util = util;
+            best = b;
+        }
     }
     return best;
 }
@@ -732,7 +729,7 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     // tile geometry: 256 threads = (1 << bx_log2) x by cells of the box of
     // non-solid cells
     const int ex = hi[0] - lo[0] + 1, ey = hi[1] - lo[1] + 1, ez = hi[2] - lo[2] + 1;
-    const int bxl = pick_bx_log2(ex, P.flags_needed);
+    const int bxl = pick_bx_log2(ex);
     c->g.nx = L.nx;
     c->g.ny = L.ny;
     c->g.nz = L.nz;
