@@ -652,6 +652,17 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     L.nx = L.w[0] ? L.ux : (std::max(L.ux, hi[0] - lo[0] + 3) + line - 1) / line * line;
     L.ny = L.uy + 2 * L.py;
     L.nz = L.uz + 2 * L.pz;
+    // Rows of 15, 17 or 20 lines take one more, by measurement: they lose where planes
+    // are powers of two.  us a step with / without the line more (and with a line of
+    // halo of its own): duct 512 x 256 x 256, FP32 1629 / 1712 (1630); 448 x 128 x 128,
+    // FP32 332 / 351 (338); 608 x 128 x 128, FP32 441 / 449 (443); 256 x 128 x 128, FP64
+    // 389 / 408 (400); elsewhere it costs under 2 % (512 x 192 x 128, FP32 594 / 585).
+    // The other lengths up to 25 lines lose up to 10 % with it (480 x 128 x 128 381 / 344).
+    // Not where the plane would pass 2 GiB, towards the limit below.
+    const int row_lines = L.nx / line;
+    if (!L.w[0] && (row_lines == 15 || row_lines == 17 || row_lines == 20) &&
+        (size_t)(L.nx + line) * L.ny * L.nz * elem <= ((size_t)1 << 31))
+        L.nx += line;
     // the last row's cells and right halo may lie past its pitch
     const size_t N = (size_t)L.nx * L.ny * L.nz +
                      (L.w[0] ? 0 : (size_t)std::max(0, L.px + std::max(L.ux, hi[0] + 2) - L.nx));
