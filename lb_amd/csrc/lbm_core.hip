@@ -617,6 +617,15 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     L.w[2] = d->periodic[2] != 0;
     const size_t elem = d->storage == LBM_STORAGE_F64 ? 8 : d->storage == LBM_STORAGE_F32 ? 4 : 2;
     const int line = (int)(128 / elem);   // populations per 128-byte cache line
+    L.py = L.w[1] ? 0 : 1;
+    L.pz = L.w[2] ? 0 : 1;
+    // too large for 32-bit plane offsets whatever the flags hold: refused before they are read
+    auto too_large = [&](size_t n) { return n * elem > 0xFFFFFFFFull || n >= 0x7FFFFFFFull; };
+    const size_t rows = ((size_t)L.uy + 2 * L.py) * ((size_t)L.uz + 2 * L.pz);
+    const size_t least = L.w[0] ? L.ux : ((size_t)L.ux + line - 1) / line * line;
+    if (rows >= 0x7FFFFFFFull || too_large(least * rows)) return LBM_E_ARG;
+    L.ny = L.uy + 2 * L.py;
+    L.nz = L.uz + 2 * L.pz;
     // Along an axis without index wrap the non-solid cells have a halo cell on
     // each side.  The box of non-solid cells, which is what the step's tiles
     // cover, starts a cache line; its left halo is the last cell of the line
@@ -647,11 +656,7 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     }
     if (L.w[0]) lo[0] -= lo[0] % line;   // no halo along x: the lattice's own lines
     L.px = L.w[0] ? 0 : line - lo[0] % line;
-    L.py = L.w[1] ? 0 : 1;
-    L.pz = L.w[2] ? 0 : 1;
     L.nx = L.w[0] ? L.ux : (std::max(L.ux, hi[0] - lo[0] + 3) + line - 1) / line * line;
-    L.ny = L.uy + 2 * L.py;
-    L.nz = L.uz + 2 * L.pz;
     // Rows of 15, 17 or 20 lines take one more, by measurement: they lose where planes
     // are powers of two.  us a step with / without the line more (and with a line of
     // halo of its own): duct 512 x 256 x 256, FP32 1629 / 1712 (1630); 448 x 128 x 128,
@@ -669,7 +674,7 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     L.n = N;
     const size_t NP = (N + line - 1) / line * line;
     const size_t NU = (size_t)L.ux * L.uy * L.uz;
-    if (N * elem > 0xFFFFFFFFull || N >= 0x7FFFFFFFull) return LBM_E_ARG;  // 32-bit plane offsets
+    if (too_large(N)) return LBM_E_ARG;
 
     Plan P;
     lbm_status st = classify(d, L, P);
