@@ -761,8 +761,9 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     c->g.ntx = (ex + (1 << bxl) - 1) >> bxl;
     c->g.nty = (ey + c->g.by - 1) / c->g.by;
     c->g.ntiles = c->g.ntx * c->g.nty * ez;
-    // a lid between walls in y, more than the L2s hold (see tile_of_block)
-    c->g.skew = c->n_upd && !L.w[1] && c->g.nty >= 8 && c->g.nty % 2 == 0 && NP * elem * Q > ((size_t)64 << 20);
+    // walls in y, more than the L2s hold (see tile_of_block)
+    c->g.skew = P.flags_needed && !L.w[1] && c->g.nty >= 8 && c->g.nty % 2 == 0 &&
+                (size_t)ex * ey * ez * elem * Q > ((size_t)64 << 20);
     c->g.tx0 = L.px + lo[0];
     c->g.ty0 = L.py + lo[1];
     c->g.tz0 = L.pz + lo[2];

@@ -282,13 +282,14 @@ __device__ __forceinline__ Cell cell_at(const Geo& g, int x, int y, int z)
 // one row group are given workgroup ids that are equal mod 8: one XCD then
 // handles the whole row group, and the odd step's x-shifted reads across a
 // tile edge find the neighbour tile's cache lines in the same L2.
-// A lid's cells are dear (each streams its own state and hands its collision over),
-// and a lid normal to y fills whole rows.  With an even number of row groups a
-// plane those rows would fall on the same one, two or four XCDs in every plane, and
-// the others wait: skew rotates the row groups by the plane's number.  258 x 130 x
-// 130 cavity, FP32: 308 -> 188 us a step; 310 x 34 x 207: 148 -> 107.  Lattices that
-// the L2s hold keep a row on one XCD from step to step instead (66^3, FP64: 27.5
-// against 28.9), and so do walls without a lid (64^3 channel, FP32: 12.2 against 14.1).
+// Cells at walls in y are dear, and a lid's dearest (each streams its own state and
+// hands its collision over); they fill whole rows.  With an even number of row
+// groups a plane those rows would fall on the same one, two or four XCDs in every
+// plane, and the others wait: skew rotates the row groups by the plane's number.  us a
+// step without / with: 258 x 130 x 130 cavity, FP32 308 / 188; 310 x 34 x 207 148 / 107;
+// channel without a lid, 256 x 258 x 256, FP16 362 / 340, FP32 643 / 645.  Lattices that
+// the L2s hold keep a row on one XCD from step to step instead (66^3 cavity, FP64
+// 27.5 / 28.9; 64^3 channel, FP32 12.2 / 14.1).
 __device__ __forceinline__ int tile_of_block(const Geo& g, int b)
 {
     if (g.ntx == 1) return b;
