@@ -519,25 +519,46 @@ static int pick_bx_log2(int nx)
 //   duct f32 384x192x160, 1316        / 588 / 566 / 574 / 568
 //   duct f16 210x101x92, 123       66 /  83 /  85 /  66 /  77
 //   duct f16 512x160x128, 617         / 284 / 277 / 290 / 284
-static void pick_cache_use(lbm_ctx* c, size_t bytes, bool rows_aligned)
+//   duct f32 200x100x104, 240           124 /     / 115 / 111 / 106
+//   duct f64 204x100x56, 240            112 /     / 112 / 104 / 103
+//   duct f32 150x100x120, 198            88 / 101 / 102 /  87 /  93
+//   duct f16 220x100x185, 244           179 /     / 170 / 165 / 166
+//   box f16 384^3, 2781               1257 /     / 1193 / 1225 / 1217
+//   box f16 320^3, 1609                 710 /     / 676 / 682 / 679
+//   box f16 288^3, 1173                 545 /     / 523 / 512 / 545
+//   channel f32 333x180x180, 1060       484 /     / 617 / 445 / 484   (rows off the lines)
+//   channel f16 333x300x300, 1471       743 /     / 1047 / 733 / 781  (rows off the lines)
+//   channel f64 203x180x180, 1292       627 /     / 859 / 577 / 646   (rows off the lines)
+//   channel f32 150x100x140, 206         83 / 159 / 164 /  84 / 114   (rows off the lines)
+//   channel f32 100x40x40, 15          14.8 / 13.9 / 13.6
+//   channel f32 50x80x60, 24           14.7 / 16.2 / 15.8             (rows off the lines)
+// bytes: of all populations; box: of those in the rows that the tiles cover.  With
+// boundaries the cache also holds classes, node words and records, and the line lies
+// at 224 MiB of the box.  Rows off the lines take no hint there: it sends partial
+// lines to memory.  (Small FP32 channels with index wrap in x do: it costs them
+// nothing in the caches of a chip that holds them whole, and they gain 4 to 8 %.)
+static void pick_cache_use(lbm_ctx* c, size_t bytes, size_t box, bool rows_aligned, bool wrap_x)
 {
     const size_t MiB = (size_t)1 << 20;
     const bool wide = c->elem >= 4;
-    c->turn = c->nt_even = c->nt_odd = false;
-    if (bytes <= 256 * MiB) return;
+    auto use = [c](bool turn, bool nt_even, bool nt_odd) {
+        c->turn = turn;
+        c->nt_even = nt_even;
+        c->nt_odd = nt_odd;
+    };
     if (c->flags_needed) {
-        c->turn = wide && bytes > 352 * MiB && bytes <= 1024 * MiB;
-        c->nt_even = !c->turn;
-        c->nt_odd = true;
-    } else if (!wide) {
-        c->turn = true;
-    } else if (!rows_aligned) {
-        c->turn = bytes > 320 * MiB;
-        c->nt_even = !c->turn;
+        if (box <= 22 * MiB && c->elem == 4 && wrap_x) use(false, true, true);
+        else if (box <= 224 * MiB) use(false, false, false);
+        else if (!rows_aligned) use(true, false, false);
+        else if (wide && box <= 1024 * MiB) use(true, false, true);
+        else use(false, true, true);
     } else {
-        c->turn = bytes <= 1024 * MiB;
-        c->nt_even = !c->turn;
-        c->nt_odd = bytes > 512 * MiB;
+        if (bytes <= 256 * MiB) use(false, false, false);
+        else if (!wide && rows_aligned && bytes > 1536 * MiB) use(false, true, true);
+        else if (!wide) use(true, false, false);
+        else if (!rows_aligned) use(bytes > 320 * MiB, bytes <= 320 * MiB, false);
+        else if (bytes <= 1024 * MiB) use(true, false, bytes > 512 * MiB);
+        else use(false, true, true);
     }
 }
 
@@ -778,7 +799,7 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     c->g.tex = ex;
     c->g.tey = ey;
     const bool rows_aligned = (size_t)L.nx * elem % 128 == 0;
-    pick_cache_use(c, NP * elem * Q, rows_aligned);
+    pick_cache_use(c, NP * elem * Q, (size_t)L.nx * ey * ez * elem * Q, rows_aligned, L.w[0]);
     // consecutive cells where the rows leave lanes idle or start inside a line
     c->g.flat = !P.flags_needed && (ex % (1 << bxl) != 0 || ey % c->g.by != 0 || !rows_aligned);
     c->g.rnx = (uint32_t)((1ull << 32) / (uint64_t)L.nx);
