@@ -613,8 +613,7 @@ __device__ __forceinline__ void step_cells(const StepArgs<ST>& a)
 // even FP32 step through step_cells computes all 27 post-collision values
 // before its stores (107 VGPRs) and ran 2.9 % faster on the periodic 256^3
 // workload (cumulant 2017: 3.2 %), while the 16-bit steps ran 2.1-2.6 %
-// slower that way and FP64 0.5 %.  No launch bound holds the 16-bit steps to more
-// waves: a hint for 7 made BGK and the 2017 operators spill 650 bytes a lane.
+// slower that way and FP64 0.5 %.
 template <class ST, int COLL, bool LIT, bool ODD, bool FLAGS, bool CC, bool INL, bool NT>
 __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
 {
@@ -623,6 +622,20 @@ __global__ __launch_bounds__(TPB) void k_step(StepArgs<ST> a)
     } else {
 #include "step_body.inc"
     }
+}
+
+// The hinted step of a lattice with boundaries in 16-bit storage, 2015 operator, held
+// to 7 waves per SIMD (72 VGPRs instead of 75, which allow 6): a 16-bit wave moves
+// half the bytes of an FP32 one, so more waves are wanted where the lattice goes to
+// memory.  us a step without / with: duct 256 x 128 x 128, FP16 153 / 146; 512 x 256 x
+// 256, BF16 994 / 945.  Lattices that the cache holds do not gain (210 x 101 x 92, FP16
+// with stochastic rounding 78.6 / 81.1), BGK and the 2017 operators spill 650 bytes a
+// lane there, and the step with the lid's rule spills all it holds (256^3 cavity, BF16
+// with stochastic rounding 465 / 4505).
+template <class ST, bool ODD>
+__global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(7, 7))) void k_step_w7(StepArgs<ST> a)
+{
+    step_cells<ST, LBM_COLLISION_CUM2015, false, ODD, true, false, false, true>(a);
 }
 
 // Moments, Smagorinsky rate and closure features of one cell, shared by the

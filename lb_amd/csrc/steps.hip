@@ -10,10 +10,16 @@
 template <class ST, int COLL, bool LIT, bool FLAGS, bool CC, bool INL>
 static void launch_step(bool odd, bool nt, dim3 grid, hipStream_t s, const StepArgs<ST>& a)
 {
-    if (odd && nt) k_step<ST, COLL, LIT, true, FLAGS, CC, INL, true><<<grid, TPB, 0, s>>>(a);
-    else if (odd) k_step<ST, COLL, LIT, true, FLAGS, CC, INL, false><<<grid, TPB, 0, s>>>(a);
-    else if (nt) k_step<ST, COLL, LIT, false, FLAGS, CC, INL, true><<<grid, TPB, 0, s>>>(a);
-    else k_step<ST, COLL, LIT, false, FLAGS, CC, INL, false><<<grid, TPB, 0, s>>>(a);
+    if (!nt) {
+        if (odd) k_step<ST, COLL, LIT, true, FLAGS, CC, INL, false><<<grid, TPB, 0, s>>>(a);
+        else k_step<ST, COLL, LIT, false, FLAGS, CC, INL, false><<<grid, TPB, 0, s>>>(a);
+    } else if constexpr (sizeof(typename ST::T) == 2 && COLL == LBM_COLLISION_CUM2015 && FLAGS && !CC && !INL) {
+        if (odd) k_step_w7<ST, true><<<grid, TPB, 0, s>>>(a);
+        else k_step_w7<ST, false><<<grid, TPB, 0, s>>>(a);
+    } else {
+        if (odd) k_step<ST, COLL, LIT, true, FLAGS, CC, INL, true><<<grid, TPB, 0, s>>>(a);
+        else k_step<ST, COLL, LIT, false, FLAGS, CC, INL, true><<<grid, TPB, 0, s>>>(a);
+    }
 }
 
 template <class ST, int COLL, bool FLAGS>
