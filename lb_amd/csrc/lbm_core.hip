@@ -993,7 +993,7 @@ lbm_status lbm_moment_avg(lbm_ctx* c, double* rho, double* ux, double* uy, doubl
     double* outs[4] = {rho, ux, uy, uz};
     // momentAvg (MomentTimeAvg.h:47-77): the sums divided by the counter
     const double n = (double)c->avg_count;
-    if (ring_ready(c, 4)) return read_planes(c, c->avg, outs, 4, n);
+    if (ring_ready(c, outs, 4)) return read_planes(c, c->avg, outs, 4, n);
     for (int k = 0; k < 4; ++k)
         if (outs[k])
             HIPCHK(hipMemcpyAsync(outs[k], c->avg + k * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost,
@@ -1073,7 +1073,7 @@ lbm_status lbm_get_macroscopic(lbm_ctx* c, double* rho, double* ux, double* uy, 
     lbm_status st = lbm_sync(c);
     if (st != LBM_OK && st != LBM_E_NAN) return st;
     double* outs[4] = {rho, ux, uy, uz};
-    if (ring_ready(c, 4))
+    if (ring_ready(c, outs, 4))
         return with_storage(c, [&](auto stv) -> lbm_status {
             using ST = decltype(stv);
             using R = typename ST::R;
@@ -1178,7 +1178,7 @@ lbm_status lbm_get_omega(lbm_ctx* c, double* omega)
         st = run_macro(c);
     }
     if (st != LBM_OK) return st;
-    if (ring_ready(c, 1)) return read_planes(c, c->stage + 4 * c->NU, &omega, 1);
+    if (ring_ready(c, &omega, 1)) return read_planes(c, c->stage + 4 * c->NU, &omega, 1);
     HIPCHK(hipMemcpyAsync(omega, c->stage + 4 * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1252,7 +1252,7 @@ lbm_status lbm_get_population(lbm_ctx* c, int32_t q, double* f)
         return LBM_OK;
     });
     if (st != LBM_OK) return st;
-    if (ring_ready(c, 1)) return read_planes(c, c->stage, &f, 1);
+    if (ring_ready(c, &f, 1)) return read_planes(c, c->stage, &f, 1);
     HIPCHK(hipMemcpyAsync(f, c->stage, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1275,7 +1275,7 @@ lbm_status lbm_get_populations(lbm_ctx* c, double* f)
         });
         if (st != LBM_OK) return st;
         double* fq = f + (size_t)q * c->NU;
-        if (ring_ready(c, 1)) {
+        if (ring_ready(c, &fq, 1)) {
             st = read_planes(c, c->stage, &fq, 1);
             if (st != LBM_OK) return st;
             continue;

@@ -26,8 +26,13 @@
 // took 17.8 ms without the ring and 20.5 with it, the 203x97x131 box (82 MB) 16.3 and
 // 24.6; the 256^3 box (537 MB) 251 and 227, the 160x144x160 FP64 box (118 MB) 52.5 and
 // 47.1.
-static inline bool ring_ready(lbm_ctx* c, int np)
+static inline bool ring_ready(lbm_ctx* c, double* const* dst, int np)
 {
+    // planes that share memory keep the order of the copies, the last one's values:
+    // the ring's threads would write them in any order
+    for (int k = 0; k < np; ++k)
+        for (int l = 0; l < k; ++l)
+            if (dst[k] && dst[l] && dst[l] < dst[k] + c->NU && dst[k] < dst[l] + c->NU) return false;
     const size_t bytes = (size_t)np * c->NU * sizeof(double);
     if (bytes > RB_SLOT && bytes < RB_MANY) return false;
     if (c->rb_host) return true;
