@@ -18,7 +18,7 @@ using namespace lbm;
 static constexpr int RB_SLOTS = 16;
 static constexpr size_t RB_SLOT = 1 << 20;
 static constexpr size_t RB_PER_THREAD = 2 << 20;
-static constexpr size_t RB_MANY = 96 << 20;   // the ring's threads are used from here on
+static constexpr size_t RB_MANY = 256 << 20;   // the ring's threads are used from here on
 
 struct lbm_ctx {
     lbm_desc d;

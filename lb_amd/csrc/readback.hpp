@@ -5,8 +5,8 @@
 // array.  Here chunks go through a ring of pinned slots, and several threads
 // move them on, so that the link, the page faults and the copies overlap; the
 // planes cross the link in the arithmetic type (the widening to FP64 is exact).
-// Four fields: 256^3 FP32 53.6 -> 10.4 ms, 192^3 FP16 21 -> 5.0, 160 x 144 x 160
-// FP64 6.7 -> 4.2 (the link's 28 GB/s), 32^3 FP32 (one slot, one thread) 0.19 -> 0.08.
+// Four fields: 256^3 FP32 41-53 -> 11 ms (the link's 28 GB/s), 32^3 FP32 (one slot,
+// one thread) 0.11 -> 0.08.
 #pragma once
 
 #include <algorithm>
@@ -18,14 +18,17 @@
 #include "context.hpp"
 
 // True where np planes go through the ring, which the first such read of a
-// context allocates (false too if there is no pinned memory): where one slot holds
-// them, which takes no other thread, and from 96 MiB on.  Between, the copies into
-// the caller's memory stay: a caller's own thread pool that spins on every CPU
-// between its uses (OpenMP's default) was held up for some 10 ms after the ring's
-// threads had run.  With such a pool, a pass of the 130x98x114 cavity (46 MB)
-// took 17.8 ms without the ring and 20.5 with it, the 203x97x131 box (82 MB) 16.3 and
-// 24.6; the 256^3 box (537 MB) 251 and 227, the 160x144x160 FP64 box (118 MB) 52.5 and
-// 47.1.
+// context allocates (false too if there is no pinned memory).
+// Outputs of at least RB_MANY bytes take the ring, and those that one slot holds,
+// which takes no other thread.  Between, the copies into the caller's memory stay: with
+// a caller's own thread pool that spins on every CPU between its uses (OpenMP's
+// default, the process's share of the CPUs no larger than the pool), one pass in ten
+// or more stalled for 10 to 30 ms after such a read.  ms a read and the pool's next use,
+// median and 90 % line, copies / ring: 256x128x128 FP32 (128 MiB) 8.5, 8.7 / 4.2, 29.8;
+// 192^3 FP32 (216) 23.4, 26.5 / 7.0, 32.2; 208^3 FP32 (275) 36.6, 37.6 / 13.9, 15.8, FP16
+// 32.4, 33.2 / 8.0, 8.4; 256^3 FP32 (512) 65.6, 69.0 / 25.0, 27.2.  The line is between the
+// largest output that stalled and the smallest that did not, at 30 to 300 steps between
+// the reads; why larger ones do not was not found.
 static inline bool ring_ready(lbm_ctx* c, double* const* dst, int np)
 {
     // planes that share memory keep the order of the copies, the last one's values:
