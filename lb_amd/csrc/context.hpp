@@ -13,11 +13,9 @@
 
 using namespace lbm;
 
-// pinned ring of the read-backs (readback.hpp): most slots, bytes of a slot,
-// bytes that another thread is worth
+// pinned ring of the read-backs (readback.hpp): its slots, bytes of a slot
 static constexpr int RB_SLOTS = 16;
 static constexpr size_t RB_SLOT = 1 << 20;
-static constexpr size_t RB_PER_THREAD = 2 << 20;
 static constexpr size_t RB_MANY = 256 << 20;   // the ring's threads are used from here on
 
 struct lbm_ctx {
@@ -88,8 +86,6 @@ struct lbm_ctx {
     // per-block partials of a diagnostics step go here instead of `partials` when set
     double* diag_dst = nullptr;
     // read-backs
-    char* rb_host = nullptr;          // pinned, rb_slots slots of RB_SLOT bytes
-    int rb_slots = 0;
     hipEvent_t rb_ev[RB_SLOTS] = {};
     // asynchronous snapshots: rho, u, omega into snap_dev on the context stream,
     // then a copy to pinned host memory on copy_stream while steps go on

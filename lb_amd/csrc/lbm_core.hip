@@ -593,7 +593,6 @@ void lbm_destroy(lbm_ctx* c)
         if (b) (void)hipFree(b);
     if (c->snap_pending && c->ev_snap_copy) (void)hipEventSynchronize(c->ev_snap_copy);
     if (c->snap_host) (void)hipHostFree(c->snap_host);
-    if (c->rb_host) (void)hipHostFree(c->rb_host);
     for (hipEvent_t e : c->rb_ev)
         if (e) (void)hipEventDestroy(e);
     if (c->ev_snap) (void)hipEventDestroy(c->ev_snap);
@@ -603,6 +602,7 @@ void lbm_destroy(lbm_ctx* c)
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    pinned_blocks().closed();
 }
 
 lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
@@ -709,6 +709,7 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
 
     lbm_ctx* c = new (std::nothrow) lbm_ctx();
     if (!c) return LBM_E_OOM;
+    pinned_blocks().opened();
     c->d = *d;
     c->d.flags = nullptr;
     c->d.bc = nullptr;
@@ -993,7 +994,7 @@ lbm_status lbm_moment_avg(lbm_ctx* c, double* rho, double* ux, double* uy, doubl
     double* outs[4] = {rho, ux, uy, uz};
     // momentAvg (MomentTimeAvg.h:47-77): the sums divided by the counter
     const double n = (double)c->avg_count;
-    if (ring_ready(c, outs, 4)) return read_planes(c, c->avg, outs, 4, n);
+    if (Ring ring(c, outs, 4); ring) return read_planes(c, ring, c->avg, outs, 4, n);
     for (int k = 0; k < 4; ++k)
         if (outs[k])
             HIPCHK(hipMemcpyAsync(outs[k], c->avg + k * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost,
@@ -1073,13 +1074,13 @@ lbm_status lbm_get_macroscopic(lbm_ctx* c, double* rho, double* ux, double* uy, 
     lbm_status st = lbm_sync(c);
     if (st != LBM_OK && st != LBM_E_NAN) return st;
     double* outs[4] = {rho, ux, uy, uz};
-    if (ring_ready(c, outs, 4))
+    if (Ring ring(c, outs, 4); ring)
         return with_storage(c, [&](auto stv) -> lbm_status {
             using ST = decltype(stv);
             using R = typename ST::R;
             k_macro<ST, R><<<blocks_for(c->NU), TPB, 0, c->stream>>>(aux_args<ST>(c));
             HIPCHK(hipGetLastError());
-            return read_planes(c, (const R*)c->stage, outs, 4);
+            return read_planes(c, ring, (const R*)c->stage, outs, 4);
         });
     st = run_macro(c);
     if (st != LBM_OK) return st;
@@ -1178,7 +1179,7 @@ lbm_status lbm_get_omega(lbm_ctx* c, double* omega)
         st = run_macro(c);
     }
     if (st != LBM_OK) return st;
-    if (ring_ready(c, &omega, 1)) return read_planes(c, c->stage + 4 * c->NU, &omega, 1);
+    if (Ring ring(c, &omega, 1); ring) return read_planes(c, ring, c->stage + 4 * c->NU, &omega, 1);
     HIPCHK(hipMemcpyAsync(omega, c->stage + 4 * c->NU, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1252,7 +1253,7 @@ lbm_status lbm_get_population(lbm_ctx* c, int32_t q, double* f)
         return LBM_OK;
     });
     if (st != LBM_OK) return st;
-    if (ring_ready(c, &f, 1)) return read_planes(c, c->stage, &f, 1);
+    if (Ring ring(c, &f, 1); ring) return read_planes(c, ring, c->stage, &f, 1);
     HIPCHK(hipMemcpyAsync(f, c->stage, c->NU * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -1264,6 +1265,7 @@ lbm_status lbm_get_populations(lbm_ctx* c, double* f)
     if (!c->initialized) return LBM_E_STATE;
     lbm_status st = lbm_sync(c);
     if (st != LBM_OK && st != LBM_E_NAN) return st;
+    Ring ring(c, &f, 1);
     for (int q = 0; q < Q; ++q) {
         st = with_storage(c, [&](auto stv) -> lbm_status {
             using ST = decltype(stv);
@@ -1275,8 +1277,8 @@ lbm_status lbm_get_populations(lbm_ctx* c, double* f)
         });
         if (st != LBM_OK) return st;
         double* fq = f + (size_t)q * c->NU;
-        if (ring_ready(c, &fq, 1)) {
-            st = read_planes(c, c->stage, &fq, 1);
+        if (ring) {
+            st = read_planes(c, ring, c->stage, &fq, 1);
             if (st != LBM_OK) return st;
             continue;
         }

@@ -12,13 +12,81 @@
 #include <algorithm>
 #include <atomic>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <thread>
 
 #include "context.hpp"
 
-// True where np planes go through the ring, which the first such read of a
-// context allocates (false too if there is no pinned memory).
+// Pinned blocks between the reads of all contexts: allocating one takes longer than
+// a small read saves, and a program makes many lattices (32^3, first read of a
+// lattice: 0.41 ms against 0.31 with the plain copies).  At most KEEP blocks stay, and
+// none after the last context.
+class PinnedBlocks {
+public:
+    char* take(size_t bytes)
+    {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            for (int k = 0; k < n; ++k)
+                if (free_[k].bytes == bytes) {
+                    char* p = free_[k].p;
+                    free_[k] = free_[--n];
+                    return p;
+                }
+        }
+        char* p = nullptr;
+        if (hipHostMalloc((void**)&p, bytes, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        return p;
+    }
+    void give(char* p, size_t bytes)
+    {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            if (contexts > 0 && n < KEEP) {
+                free_[n++] = {p, bytes};
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+    void opened()
+    {
+        std::lock_guard<std::mutex> lock(m);
+        ++contexts;
+    }
+    void closed()
+    {
+        Block drop[KEEP];
+        int k = 0;
+        {
+            std::lock_guard<std::mutex> lock(m);
+            if (--contexts == 0)
+                while (n) drop[k++] = free_[--n];
+        }
+        while (k) (void)hipHostFree(drop[--k].p);
+    }
+
+private:
+    static constexpr int KEEP = 4;
+    struct Block {
+        char* p;
+        size_t bytes;
+    };
+    std::mutex m;
+    Block free_[KEEP];
+    int n = 0, contexts = 0;
+};
+
+static inline PinnedBlocks& pinned_blocks()
+{
+    static PinnedBlocks b;
+    return b;
+}
+
 // Outputs of at least RB_MANY bytes take the ring, and those that one slot holds,
 // which takes no other thread.  Between, the copies into the caller's memory stay: with
 // a caller's own thread pool that spins on every CPU between its uses (OpenMP's
@@ -29,36 +97,46 @@
 // 32.4, 33.2 / 8.0, 8.4; 256^3 FP32 (512) 65.6, 69.0 / 25.0, 27.2.  The line is between the
 // largest output that stalled and the smallest that did not, at 30 to 300 steps between
 // the reads; why larger ones do not was not found.
-static inline bool ring_ready(lbm_ctx* c, double* const* dst, int np)
-{
-    // planes that share memory keep the order of the copies, the last one's values:
-    // the ring's threads would write them in any order
-    for (int k = 0; k < np; ++k)
-        for (int l = 0; l < k; ++l)
-            if (dst[k] && dst[l] && dst[l] < dst[k] + c->NU && dst[k] < dst[l] + c->NU) return false;
-    const size_t bytes = (size_t)np * c->NU * sizeof(double);
-    if (bytes > RB_SLOT && bytes < RB_MANY) return false;
-    if (c->rb_host) return true;
-    // no more slots than five FP64 planes fill
-    c->rb_slots = (int)std::min<size_t>(RB_SLOTS, (5 * c->NU * sizeof(double) + RB_SLOT - 1) / RB_SLOT);
-    for (int k = 0; k < c->rb_slots; ++k)
-        if (!c->rb_ev[k] && hipEventCreateWithFlags(&c->rb_ev[k], hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            c->rb_ev[k] = nullptr;
-            return false;
+class Ring {
+public:
+    // wanted planes: dst[k] not null.  Planes that share memory keep the order of the
+    // copies, the last one's values.
+    Ring(lbm_ctx* c, double* const* dst, int np)
+    {
+        size_t wanted = 0;
+        for (int k = 0; k < np; ++k) {
+            if (!dst[k]) continue;
+            ++wanted;
+            for (int l = 0; l < k; ++l)
+                if (dst[l] && dst[l] < dst[k] + c->NU && dst[k] < dst[l] + c->NU) return;
         }
-    if (hipHostMalloc((void**)&c->rb_host, RB_SLOT * c->rb_slots, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        c->rb_host = nullptr;
-        return false;
+        const size_t bytes = wanted * c->NU * sizeof(double);
+        if (bytes > RB_SLOT && bytes < RB_MANY) return;
+        slots = bytes <= RB_SLOT ? 1 : RB_SLOTS;
+        for (int k = 0; k < slots; ++k)
+            if (!c->rb_ev[k] && hipEventCreateWithFlags(&c->rb_ev[k], hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                c->rb_ev[k] = nullptr;
+                return;
+            }
+        mem = pinned_blocks().take(slots * RB_SLOT);
     }
-    return true;
-}
+    ~Ring()
+    {
+        if (mem) pinned_blocks().give(mem, slots * RB_SLOT);
+    }
+    Ring(const Ring&) = delete;
+    Ring& operator=(const Ring&) = delete;
+    explicit operator bool() const { return mem != nullptr; }
+
+    char* mem = nullptr;
+    int slots = 0;
+};
 
 // np planes of c->NU values each, consecutive at src, divided by div, to dst[k]
 // (null: not wanted).  Returns when they have arrived.
 template <class S>
-static lbm_status read_planes(lbm_ctx* c, const S* src, double* const* dst, int np, double div = 1.0)
+static lbm_status read_planes(lbm_ctx* c, const Ring& ring, const S* src, double* const* dst, int np, double div = 1.0)
 {
     // a chunk: values [i, i + n) of the planes' run, which may be of several planes
     struct Chunk {
@@ -82,8 +160,8 @@ static lbm_status read_planes(lbm_ctx* c, const S* src, double* const* dst, int 
     std::atomic<int> issued{0}, claimed{0};
     std::atomic<bool> failed{false};
 
-    const int K = c->rb_slots;
-    auto slot = [&](int j) { return (S*)(c->rb_host + (size_t)(j % K) * RB_SLOT); };
+    const int K = ring.slots;
+    auto slot = [&](int j) { return (S*)(ring.mem + (size_t)(j % K) * RB_SLOT); };
     auto move = [&](int j) {
         if (hipEventSynchronize(c->rb_ev[j % K]) != hipSuccess) {
             failed = true;
@@ -113,10 +191,9 @@ static lbm_status read_planes(lbm_ctx* c, const S* src, double* const* dst, int 
             move(j);
         }
     };
-    // one thread more for every 2 MB, up to 7
+    // a small output takes no other thread, a large one up to 7
     std::vector<std::thread> team;
-    const int nt = (int)std::min<size_t>({7, std::max(2u, std::thread::hardware_concurrency()) / 2 - 1,
-                                          (size_t)n * RB_SLOT / RB_PER_THREAD});
+    const int nt = K == 1 ? 0 : (int)std::min<size_t>({7, std::max(4u, std::thread::hardware_concurrency()) / 2 - 1, (size_t)n - 1});
     try {
         team.reserve(nt);
         for (int t = 0; t < nt; ++t) team.emplace_back(worker);

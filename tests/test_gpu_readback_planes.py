@@ -60,3 +60,26 @@ def test_planes_in_shared_memory(n):
     assert np.array_equal(both[:half], full[2].ravel()[:half])
     assert np.array_equal(both[half:half + a.size], full[3].ravel())
     L.close()
+
+
+def test_lattices_of_several_threads_share_the_pinned_blocks():
+    import threading
+    for _ in range(2):   # the second round starts without a context: the blocks were given back
+        bad = []
+
+        def work(k):
+            L = Lattice(make_desc(np.ones((16, 20, 24), np.int32), [], storage=abi.STORAGE_F64, arith=abi.ARITH_FAST,
+                                  periodic=(1, 1, 1), tau=0.6))
+            rho = 1.0 + 0.01 * (k + np.random.default_rng(k).random((16, 20, 24)))
+            L.init_equilibrium(rho, None, None, None)
+            for _ in range(40):
+                if not np.array_equal(L.macroscopic()[0], rho):
+                    bad.append(k)
+            L.close()
+
+        team = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+        for t in team:
+            t.start()
+        for t in team:
+            t.join()
+        assert not bad
