@@ -532,11 +532,22 @@ static int pick_bx_log2(int nx)
 //   channel f32 150x100x140, 206         83 / 159 / 164 /  84 / 114   (rows off the lines)
 //   channel f32 100x40x40, 15          14.8 / 13.9 / 13.6
 //   channel f32 50x80x60, 24           14.7 / 16.2 / 15.8             (rows off the lines)
+//   cavity f32 310x34x207, 216          106 /     /  96 /  93 /  93
+//   duct f64 200x100x49, 206             85 /     /  98 /  85 /  91
+//   box f16 32x90x122, 18              14.0 / 12.4 / 12.3             (rows off the lines)
+//   box bf16 128x98x33, 21             15.3 /     / 13.2
+//   box f16 40^3, 3                     5.9 / 6.1 / 6.3               (rows off the lines)
+//   box f32 64^3, 27                   10.8 / 10.3 / 10.1
+//   box f32 62x61x65, 25               12.4 / 12.5 / 13.6             (rows off the lines)
+//   box f64 64x78x23, 24               10.6 /     / 12.0
+//   channel f64 83x58x29, 29           12.8 /     / 15.8              (rows off the lines)
+//   cavity f16 40^3, 3                 10.7 / 11.5 / 11.5
 // bytes: of all populations; box: of those in the rows that the tiles cover.  With
 // boundaries the cache also holds classes, node words and records, and the line lies
-// at 224 MiB of the box.  Rows off the lines take no hint there: it sends partial
-// lines to memory.  (Small FP32 channels with index wrap in x do: it costs them
-// nothing in the caches of a chip that holds them whole, and they gain 4 to 8 %.)
+// at 208 MiB of the box.  Rows off the lines take no hint there: it sends partial
+// lines to memory.  What the L2s hold (8 to 22 MiB, FP32 and 16-bit rows on the lines
+// to 28) takes it, where x has index wrap: it costs nothing there, and boxes and
+// channels gain up to 14 % (cavities lose by it).
 static void pick_cache_use(lbm_ctx* c, size_t bytes, size_t box, bool rows_aligned, bool wrap_x)
 {
     const size_t MiB = (size_t)1 << 20;
@@ -546,9 +557,10 @@ static void pick_cache_use(lbm_ctx* c, size_t bytes, size_t box, bool rows_align
         c->nt_even = nt_even;
         c->nt_odd = nt_odd;
     };
-    if (c->flags_needed) {
-        if (box <= 22 * MiB && c->elem == 4 && wrap_x) use(false, true, true);
-        else if (box <= 224 * MiB) use(false, false, false);
+    if (wrap_x && box > 8 * MiB && box <= (c->elem <= 4 && rows_aligned ? 28 : 22) * MiB) {
+        use(false, true, true);
+    } else if (c->flags_needed) {
+        if (box <= 208 * MiB) use(false, false, false);
         else if (!rows_aligned) use(true, false, false);
         else if (wide && box <= 1024 * MiB) use(true, false, true);
         else use(false, true, true);
