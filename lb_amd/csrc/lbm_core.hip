@@ -813,8 +813,12 @@ lbm_status lbm_create(const lbm_desc* d, lbm_ctx** out)
     c->g.tey = ey;
     const bool rows_aligned = (size_t)L.nx * elem % 128 == 0;
     pick_cache_use(c, NP * elem * Q, (size_t)L.nx * ey * ez * elem * Q, rows_aligned, L.w[0]);
-    // consecutive cells where the rows leave lanes idle or start inside a line
-    c->g.flat = !P.flags_needed && (ex % (1 << bxl) != 0 || ey % c->g.by != 0 || !rows_aligned);
+    // consecutive cells where the rows leave lanes idle or start inside a line; not
+    // where the row tiles are no more than the CUs, whose idle lanes cost nothing (FP64,
+    // us a step with row tiles / consecutive cells: 48 x 31 x 29 6.7 / 8.3, 31 x 59 x 26
+    // 7.2 / 8.4, 64 x 33 x 23 8.1 / 6.7)
+    c->g.flat = !P.flags_needed && c->g.ntiles > 256 &&
+                (ex % (1 << bxl) != 0 || ey % c->g.by != 0 || !rows_aligned);
     c->g.rnx = (uint32_t)((1ull << 32) / (uint64_t)L.nx);
     c->g.rny = (uint32_t)((1ull << 32) / (uint64_t)L.ny);
     if (c->g.flat) c->g.ntiles = (int)blocks_for(NU);
