@@ -542,6 +542,7 @@ static int pick_bx_log2(int nx)
 //   box f64 64x78x23, 24               10.6 /     / 12.0
 //   channel f64 83x58x29, 29           12.8 /     / 15.8              (rows off the lines)
 //   cavity f16 40^3, 3                 10.7 / 11.5 / 11.5
+// (f16 192^3, 256^3, 210x101x92 and 512x160x128 with a collision of fewer instructions.)
 // bytes: of all populations; box: of those in the rows that the tiles cover.  With
 // boundaries the cache also holds classes, node words and records, and the line lies
 // at 208 MiB of the box.  Rows off the lines take no hint there: it sends partial
